@@ -93,7 +93,10 @@ typedef struct kvmc_desc {
     int32_t refresh_k;      /* accepted moves per refresh for EVERY_K */
     int32_t delay;          /* pending rank-1 updates kept before one rank-`delay`
                                flush of W (<= 1: immediate, as the reference);
-                               FP32 and FP64 alike */
+                               FP32 and FP64 alike.  FP64 handles may keep
+                               terms of their own for immediate updates: the
+                               same W to rounding, and each accepted move
+                               counts as a flush */
     int32_t threads;        /* threads per workgroup of the sweep kernel (0: auto) */
     uint64_t seed;          /* Philox key of the device RNG */
     int32_t orbitals;       /* KVMC_ORB_* */

@@ -173,6 +173,7 @@ struct kvmc_handle {
     int ns = 0, nup = 0, ndn = 0, nb = 0, nmax = 0, nsp = 0;
     int nw = 0;
     int prec = 0, kernel = 0, policy = 0, refresh_k = 0, delay = 1, threads = 0;
+    int asked_delay = 1;            // the descriptor's; `delay` is what the kernels keep pending
     int cplx = 0;                   // complex orbitals: W in complex float / double
     uint64_t seed = 0;
     size_t esize = 8;
@@ -205,6 +206,7 @@ struct kvmc_handle {
     int* zmu = nullptr;
     int* acc_since = nullptr;
     int* status = nullptr;
+    int* stiff = nullptr;           // [nw][2] nearly singular tildeU at the last refresh
     long long* sweeps = nullptr;
     long long* stop = nullptr;
     long long* tbase = nullptr;
@@ -249,7 +251,7 @@ namespace {
 void free_all(kvmc_handle* h) {
     void* ptrs[] = {h->bonds, h->nbr_off, h->nbr, h->Uup, h->Udn, h->UTup, h->UTdn, h->Ucup, h->Ucdn, h->kRup,
                     h->kRdn, h->eloc_im, h->kup, h->kdn, h->W, h->slot, h->A,
-                    h->Bm, h->npend, h->pterm, h->zmu, h->acc_since, h->status, h->sweeps, h->stop,
+                    h->Bm, h->npend, h->pterm, h->zmu, h->acc_since, h->status, h->stiff, h->sweeps, h->stop,
                     h->tbase, h->rlist, h->rcount, h->failed, h->all_walkers, h->counters,
                     h->logdet, h->eloc, h->drift, h->dstats, h->ws, h->Qup, h->Qdn, h->O};
     for (void* p : ptrs)
@@ -282,7 +284,7 @@ SweepArgs sweep_args(kvmc_handle* h) {
     a.bonds = h->bonds; a.nbr_off = h->nbr_off; a.nbr = h->nbr;
     a.kup = h->kup; a.kdn = h->kdn; a.W = h->W; a.slot = h->slot; a.A = h->A; a.Bm = h->Bm;
     a.npend = h->npend; a.delay = h->delay; a.nmax = h->nmax;
-    a.pterm = h->pterm;
+    a.pterm = h->pterm; a.stiff = h->stiff;
     a.sweeps = h->sweeps; a.stop = h->stop; a.tape_base = h->tbase;
     a.zmu = h->zmu; a.acc_since = h->acc_since;
     a.refresh_list = h->rlist; a.refresh_count = h->rcount;
@@ -303,7 +305,7 @@ RefreshArgs refresh_args(const kvmc_handle* h, int write_w, double pivot_tol) {
     r.npend = h->npend; r.acc_since = h->acc_since; r.delay = h->delay; r.nmax = f * h->nmax;
     r.ns_out = h->ns; r.nup_out = h->nup; r.ndn_out = h->ndn; r.nmax_out = h->nmax; r.cplx_out = h->cplx;
     r.ws = h->ws; r.logdet = h->logdet; r.status = h->status; r.failed = h->failed;
-    r.write_w = write_w; r.drift = h->drift; r.pivot_tol = pivot_tol;
+    r.write_w = write_w; r.stiff = h->stiff; r.drift = h->drift; r.pivot_tol = pivot_tol;
     return r;
 }
 
@@ -449,7 +451,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
         return fail(KVMC_ERR_INVALID, "unknown refresh policy");
     if (d->refresh_policy != KVMC_REFRESH_REFERENCE && d->refresh_k <= 0)
         return fail(KVMC_ERR_INVALID, "refresh_k must be positive");
-    const int delay = d->delay <= 1 ? 1 : d->delay;
+    int delay = d->delay <= 1 ? 1 : d->delay;
     if (delay > kMaxDelay)
         return fail(KVMC_ERR_INVALID, "delay must be <= " + std::to_string(kMaxDelay));
     if (d->orbitals != KVMC_ORB_REAL && d->orbitals != KVMC_ORB_COMPLEX)
@@ -472,6 +474,10 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     h->prec = d->precision; h->kernel = d->kernel; h->policy = d->refresh_policy;
     h->refresh_k = d->refresh_k; h->delay = delay; h->threads = d->threads; h->seed = d->seed;
     h->cplx = d->orbitals == KVMC_ORB_COMPLEX ? 1 : 0;
+    h->asked_delay = delay;
+    // FP64 with immediate updates: the same W to rounding from pending terms
+    if (h->prec == KVMC_PREC_FP64 && delay == 1)
+        h->delay = delay = sweep_ib_fp64_delay(h->cplx, h->ns, h->nup, h->ndn, h->nb);
     h->esize = w_elem_bytes(h->prec, h->cplx);
     (void)hipGetDevice(&h->device);
     int rc = KVMC_OK;
@@ -510,7 +516,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
         ALLOC(p, nw * 2 * pend_ld(delay) * (size_t)w_nsa(h->ns, h->nup, h->ndn) * h->esize); h->A = p;
         ALLOC(p, nw * 2 * pend_ld(delay) * h->nmax * h->esize); h->Bm = p;
     }
-    ALLOC(h->npend, nw); ALLOC(h->pterm, nw * 2 * kMaxDelay * 2); ALLOC(h->zmu, nw); ALLOC(h->acc_since, nw); ALLOC(h->status, nw);
+    ALLOC(h->npend, nw); ALLOC(h->pterm, nw * 2 * kMaxDelay * 2); ALLOC(h->zmu, nw); ALLOC(h->acc_since, nw); ALLOC(h->status, nw); ALLOC(h->stiff, 2 * nw);
     ALLOC(h->sweeps, nw); ALLOC(h->stop, nw); ALLOC(h->tbase, nw);
     ALLOC(h->rlist, nw); ALLOC(h->rcount, 1); ALLOC(h->failed, 1); ALLOC(h->all_walkers, nw);
     ALLOC(h->counters, (size_t)CNT_SLOTS);
@@ -581,6 +587,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
         up(h->all_walkers, allw.data(), nw * sizeof(int)) != hipSuccess ||
         hipMemsetAsync(h->sweeps, 0, nw * sizeof(long long), h->stream) != hipSuccess ||
         hipMemsetAsync(h->npend, 0, nw * sizeof(int), h->stream) != hipSuccess ||
+        hipMemsetAsync(h->stiff, 0, 2 * nw * sizeof(int), h->stream) != hipSuccess ||
         hipMemsetAsync(h->acc_since, 0, nw * sizeof(int), h->stream) != hipSuccess ||
         hipMemsetAsync(h->logdet, 0, 2 * nw * sizeof(double), h->stream) != hipSuccess ||
         hipMemsetAsync(h->dstats, 0, 3 * sizeof(double), h->stream) != hipSuccess ||
@@ -789,7 +796,8 @@ int sweep_tail(kvmc_handle* h, const SweepArgs& a, int threads, size_t lds, bool
         counters->moves = (int64_t)cnt[CNT_MOVES];
         counters->accepted = (int64_t)cnt[CNT_ACCEPTED];
         counters->refreshes = (int64_t)cnt[CNT_PAUSES];
-        counters->flushes = (int64_t)cnt[CNT_FLUSHES];
+        // immediate updates: each accepted move updates W, whatever is kept pending
+        counters->flushes = (int64_t)cnt[h->asked_delay > 1 ? CNT_FLUSHES : CNT_ACCEPTED];
         counters->launches = launches;
     }
     return KVMC_OK;
@@ -814,7 +822,7 @@ int sweep_staged(kvmc_handle* h, int64_t nsweeps, const double* tape_u, const in
     a.outcomes = outcomes ? d_out : nullptr;
     a.walker0 = 0;
     const int threads = sweep_threads(h);
-    const size_t lds = sweep_lds_bytes(h->esize, h->ns, h->nup, h->ndn, h->delay, h->nb);
+    const size_t lds = sweep_lds_bytes(h->esize, h->ns, h->nup, h->ndn, h->asked_delay, h->nb);
     if (lds > 160 * 1024) return fail(KVMC_ERR_INVALID, "LDS footprint exceeds 160 KiB; lower delay");
     int64_t launches = 0;
     hipStream_t s = h->stream;
@@ -963,7 +971,7 @@ int kvmc_group_sweep(kvmc_group* g, const int64_t* nsweeps, kvmc_counters* count
         kvmc_handle* h = g->hs[i];
         args[i] = sweep_args(h);
         threads[i] = sweep_threads(h);
-        lds[i] = sweep_lds_bytes(h->esize, h->ns, h->nup, h->ndn, h->delay, h->nb);
+        lds[i] = sweep_lds_bytes(h->esize, h->ns, h->nup, h->ndn, h->asked_delay, h->nb);
         if (lds[i] > 160 * 1024) return fail(KVMC_ERR_INVALID, "LDS footprint exceeds 160 KiB; lower delay");
     }
     if (!g->gexec || g->g_nsweeps != std::vector<int64_t>(nsweeps, nsweeps + n)) {

@@ -9,6 +9,7 @@
 namespace kvmc {
 
 hipError_t launch_sweep_c(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
+    if (sweep_ib_supported(prec, 1, a.ns, a.nup, a.ndn, a.delay, a.nb)) return launch_sweep_ib(prec, 1, a, nw, s);
     // 16-byte vectors: two complex floats or one complex double
     if (prec == 0) return launch_sweep_v<cf64, 1>(a, nw, threads, lds, s);
     return launch_sweep_v<cf32, 2>(a, nw, threads, lds, s);

@@ -19,6 +19,10 @@ enum : int { CNT_MOVES = 0, CNT_ACCEPTED = 1, CNT_FLUSHES = 2, CNT_SWEEPS = 3, C
 // Largest number of pending rank-1 updates kept per spin before a flush.
 constexpr int kMaxDelay = 16;
 
+// Pivots of tildeU spanning more than 1e7: W has elements of that size and an
+// update of it loses as many digits (RefreshArgs::stiff).
+constexpr double kStiffTol = 1e-7;
+
 // Complex W element (complex orbitals: flux phases or a magnetic field make
 // the spinon Hamiltonian complex, src/Hamiltonian.jl:201, 325, 382-393).
 // Stored interleaved (re, im) like Julia's ComplexF64 / ComplexF32.
@@ -134,9 +138,10 @@ struct SweepArgs {
     signed char* outcomes;          // [nw][tape_len] or null
     int kernel_mode, policy, refresh_k;
     int walker0;                    // first walker of this launch
-    // FP32 sweep with implicit pending rows (k_sweep_ib): the row slot K_q
+    // sweep with implicit pending rows (k_sweep_ib): the row slot K_q
     // and label l_q of each pending term, [nw][2][kMaxDelay][2]
     int* pterm;
+    const int* stiff;               // [nw][2] the last refresh found pivots over more than 1 / kStiffTol
 };
 
 struct RefreshArgs {
@@ -164,6 +169,7 @@ struct RefreshArgs {
     int* failed;                    // smallest failing walker (atomicMin)
     int write_w;                    // 1: replace W; 0: measure drift only
     double pivot_tol;               // reject when min|pivot| < pivot_tol * max|pivot|
+    int* stiff;                     // [nw][2] min|pivot| < kStiffTol * max|pivot| (write_w)
     double* drift;                  // [nw][2] per walker: max |W_new - W_cur|, max |W_new| (ordered bits)
     // Storage shape of W, the slot map and the pending terms.  Real orbitals:
     // the same as the factorised problem.  Complex orbitals (cplx_out = 1):
@@ -208,10 +214,15 @@ hipError_t launch_sweep(int prec, const SweepArgs& a, int nwalkers, int threads,
                         hipStream_t s);
 hipError_t launch_sweep_c(int prec, const SweepArgs& a, int nwalkers, int threads, size_t lds,
                           hipStream_t s);
-// FP32 sweep with implicit pending rows (kvmc_sweep_ib.hip): real W streamed
-// from HBM, at most 256 rows per spin, 1 < delay <= kMaxDelay.
-bool sweep_ib_supported(int prec, int cplx, int ns, int nup, int ndn, int delay);
-hipError_t launch_sweep_ib(const SweepArgs& a, int nwalkers, hipStream_t s);
+// Sweep with implicit pending rows (kvmc_sweep_ib.hip): W streamed from HBM,
+// at most 256 rows per spin, 1 < delay <= kMaxDelay (8 for complex W), real
+// FP32 or any FP64.
+bool sweep_ib_supported(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb);
+// The delay FP64 handles with immediate updates (delay <= 1) run with: the
+// same W to rounding, streamed once per that many accepts; 1 where the kernel
+// does not apply.
+int sweep_ib_fp64_delay(int cplx, int ns, int nup, int ndn, int nb);
+hipError_t launch_sweep_ib(int prec, int cplx, const SweepArgs& a, int nwalkers, hipStream_t s);
 size_t sweep_lds_bytes(size_t esize, int ns, int nup, int ndn, int delay, int nb);
 // Both W of a walker at most this large: the sweep kernel keeps them in LDS.
 constexpr size_t kResidentMaxBytes = 64 * 1024;

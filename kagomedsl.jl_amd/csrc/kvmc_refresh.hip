@@ -694,6 +694,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
     }
     if (t == 0) {
         a.logdet[(size_t)w * 2 + spin] = logdet;
+        if (a.write_w) a.stiff[(size_t)w * 2 + spin] = pmin < kStiffTol * pmax;
         if (a.write_w && spin == 0) { a.npend[w] = 0; a.acc_since[w] = 0; }
     }
     if constexpr (!FULL) {
