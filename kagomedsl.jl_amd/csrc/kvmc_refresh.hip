@@ -52,11 +52,13 @@ constexpr int kStoreBlock = 8;   // sites per LDS block of the single kernel's W
 
 __host__ __device__ inline int rup_i(int x, int m) { return (x + m - 1) / m * m; }
 __host__ __device__ inline int refresh_nrows(int ns) { return rup_i(ns, 16) + 16; }
-// Register tiles per wavefront of k_refresh_solve for N <= 256: 4, 8, 14 or
-// 16 tiles of 16 labels (0: N > 256).
+// Register tiles per wavefront of k_refresh_solve for N <= 256: the next even
+// number of 16-label tiles (0: N > 256).  Tiles past the labels are zeros, but
+// cost their share of the products: with instances of 4, 8, 14 and 16 tiles
+// only, 10 tiles (N = 150) did the work of 14.
 __host__ __device__ inline int solve_nt(int nmax) {
     const int nt = (nmax + 15) / 16;
-    return nt <= 4 ? 4 : nt <= 8 ? 8 : nt <= 14 ? 14 : nt <= 16 ? 16 : 0;
+    return nt <= 16 ? (nt + 1) / 2 * 2 : 0;
 }
 // Row stride of M: whole 16 * NT rows for the solve kernel's row loads.
 __host__ __device__ inline int refresh_ldm(int nmax) { return solve_nt(nmax) ? 16 * solve_nt(nmax) : rup_i(nmax, 32); }
@@ -960,7 +962,7 @@ __device__ __forceinline__ void solve_stage(const double* M, int ldm, const int*
 // It also writes the unit rows of the occupied sites between its first
 // empty site and the next group's, so every entry of W is written once.
 template <typename T, int NT>
-__global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(NT <= 6 ? 4 : NT <= 8 ? 3 : 2)))
 k_refresh_solve(RefreshArgs a, int groups) {
     __shared__ __align__(16) double sb0[NT * 256], sb1[NT * 256];   // tile-major row blocks
     __shared__ __align__(16) double sd0[256], sd1[256];
@@ -1250,25 +1252,20 @@ static int solve_tiles(int ns, int nmax) {
 
 template <typename T>
 static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t s) {
-    switch (solve_tiles(a.ns, a.nmax)) {
-        case 4: {
-            hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
-            return e != hipSuccess ? e : launch_solve<T, 4>(a, s);
+    const int tiles = solve_tiles(a.ns, a.nmax);
+    if (tiles) {
+        hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
+        if (e != hipSuccess) return e;
+        switch (tiles) {
+            case 2: return launch_solve<T, 2>(a, s);
+            case 4: return launch_solve<T, 4>(a, s);
+            case 6: return launch_solve<T, 6>(a, s);
+            case 8: return launch_solve<T, 8>(a, s);
+            case 10: return launch_solve<T, 10>(a, s);
+            case 12: return launch_solve<T, 12>(a, s);
+            case 14: return launch_solve<T, 14>(a, s);
+            default: return launch_solve<T, 16>(a, s);
         }
-        case 8: {
-            hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
-            return e != hipSuccess ? e : launch_solve<T, 8>(a, s);
-        }
-        case 14: {
-            hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
-            return e != hipSuccess ? e : launch_solve<T, 14>(a, s);
-        }
-        case 16: {
-            hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
-            return e != hipSuccess ? e : launch_solve<T, 16>(a, s);
-        }
-        default:
-            break;
     }
     switch (refresh_rows_per_thread(a.nmax)) {
         case 1: return launch_lu<T, 1, true>(a, lds, s);
