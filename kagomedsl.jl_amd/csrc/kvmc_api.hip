@@ -105,12 +105,46 @@ void random_config(uint64_t seed, uint32_t walker, uint32_t attempt, int ns, int
     for (int b = 0; b < ndn; ++b) kdn[perm[nup + b]] = b + 1;
 }
 
-__global__ void k_set_stop(const long long* sweeps, long long* stop, long long* base,
-                           long long nsweeps, int nw) {
+// Start of a sweep call: stop counts, the walkers' counters and their sums cleared.
+__global__ void k_set_stop(const long long* sweeps, long long* stop, long long* base, long long nsweeps, int nw,
+                           unsigned long long* counters, unsigned long long* total) {
     int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w < nw) {
         base[w] = sweeps[w];
         stop[w] = sweeps[w] + nsweeps;
+        for (int q = 0; q < CNT_SLOTS; ++q) counters[(size_t)w * CNT_SLOTS + q] = 0;
+    }
+    if (w < CNT_SLOTS) total[w] = 0;
+}
+
+// total[slot] += sum over walkers of counters[walker][slot]; threads take the
+// slots in turn (blockDim a multiple of CNT_SLOTS).
+__global__ void __launch_bounds__(256) k_sum_counters(const unsigned long long* counters, unsigned long long* total, int nw) {
+    __shared__ unsigned long long part[256];
+    const int t = (int)threadIdx.x;
+    const size_t n = (size_t)nw * CNT_SLOTS, step = (size_t)gridDim.x * 256;
+    unsigned long long v = 0;
+    for (size_t q = (size_t)blockIdx.x * 256 + t; q < n; q += step) v += counters[q];
+    part[t] = v;
+    __syncthreads();
+    if (t < CNT_SLOTS) {
+        for (int q = t + CNT_SLOTS; q < 256; q += CNT_SLOTS) v += part[q];
+        atomicAdd(&total[t], v);
+    }
+}
+
+// *total = sum of nap over the walkers (one block).
+__global__ void __launch_bounds__(1024) k_sum_nap(const int* nap, unsigned long long* total, int nw) {
+    __shared__ unsigned long long part[16];
+    const int t = (int)threadIdx.x;
+    unsigned long long v = 0;
+    for (int w = t; w < nw; w += 1024) v += (unsigned long long)nap[w];
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    if (t % 64 == 0) part[t / 64] = v;
+    __syncthreads();
+    if (t == 0) {
+        for (int q = 1; q < 16; ++q) v += part[q];
+        *total = v;
     }
 }
 
@@ -120,11 +154,6 @@ __global__ void k_fill_ll(long long* p, long long v, int n) {
 }
 
 __global__ void k_fill_i(int* p, int v, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
-}
-
-__global__ void k_fill_ull(unsigned long long* p, unsigned long long v, int n) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
 }
@@ -184,6 +213,7 @@ struct kvmc_handle {
     int2* bonds = nullptr;
     int* nbr_off = nullptr;
     int* nbr = nullptr;
+    unsigned char* table = nullptr;   // the bond tables packed (bond_table_bytes)
     // U for the refresh (column-major) and its row-major copy; complex
     // orbitals: the 2 ns x 2 N real form [U_re, -U_im ; U_im, U_re]
     double* Uup = nullptr;
@@ -214,7 +244,9 @@ struct kvmc_handle {
     int* rcount = nullptr;
     int* failed = nullptr;
     int* all_walkers = nullptr;
-    unsigned long long* counters = nullptr;
+    unsigned long long* counters = nullptr;   // [nw][CNT_SLOTS] of the current sweep call
+    unsigned long long* total = nullptr;      // [CNT_SLOTS] their sums, then one slot for the sum of nap
+    int* nap = nullptr;                       // [nw] antiparallel bonds of the last measurement
     double* logdet = nullptr;
     double* eloc = nullptr;
     double* drift = nullptr;        // [nw][2] per-walker drift maxima of a drift pass
@@ -249,10 +281,10 @@ struct kvmc_group {
 namespace {
 
 void free_all(kvmc_handle* h) {
-    void* ptrs[] = {h->bonds, h->nbr_off, h->nbr, h->Uup, h->Udn, h->UTup, h->UTdn, h->Ucup, h->Ucdn, h->kRup,
+    void* ptrs[] = {h->bonds, h->nbr_off, h->nbr, h->table, h->Uup, h->Udn, h->UTup, h->UTdn, h->Ucup, h->Ucdn, h->kRup,
                     h->kRdn, h->eloc_im, h->kup, h->kdn, h->W, h->slot, h->A,
                     h->Bm, h->npend, h->pterm, h->zmu, h->acc_since, h->status, h->stiff, h->sweeps, h->stop,
-                    h->tbase, h->rlist, h->rcount, h->failed, h->all_walkers, h->counters,
+                    h->tbase, h->rlist, h->rcount, h->failed, h->all_walkers, h->counters, h->total, h->nap,
                     h->logdet, h->eloc, h->drift, h->dstats, h->ws, h->Qup, h->Qdn, h->O};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -281,7 +313,7 @@ SweepArgs sweep_args(kvmc_handle* h) {
     SweepArgs a{};
     a.ns = h->ns; a.nup = h->nup; a.ndn = h->ndn; a.nb = h->nb;
     a.nocc = std::min(h->nup, h->ndn);
-    a.bonds = h->bonds; a.nbr_off = h->nbr_off; a.nbr = h->nbr;
+    a.bonds = h->bonds; a.nbr_off = h->nbr_off; a.nbr = h->nbr; a.table = h->table;
     a.kup = h->kup; a.kdn = h->kdn; a.W = h->W; a.slot = h->slot; a.A = h->A; a.Bm = h->Bm;
     a.npend = h->npend; a.delay = h->delay; a.nmax = h->nmax;
     a.pterm = h->pterm; a.stiff = h->stiff;
@@ -488,6 +520,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     ALLOC(h->bonds, (size_t)h->nb);
     ALLOC(h->nbr_off, ns + 1);
     ALLOC(h->nbr, (size_t)2 * h->nb);
+    ALLOC(h->table, bond_table_bytes(h->ns, h->nb));
     const size_t f2 = (size_t)cf * cf;   // the real form has cf^2 times the entries
     ALLOC(h->Uup, f2 * ns * h->nup);
     ALLOC(h->Udn, f2 * ns * h->ndn);
@@ -519,7 +552,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     ALLOC(h->npend, nw); ALLOC(h->pterm, nw * 2 * kMaxDelay * 2); ALLOC(h->zmu, nw); ALLOC(h->acc_since, nw); ALLOC(h->status, nw); ALLOC(h->stiff, 2 * nw);
     ALLOC(h->sweeps, nw); ALLOC(h->stop, nw); ALLOC(h->tbase, nw);
     ALLOC(h->rlist, nw); ALLOC(h->rcount, 1); ALLOC(h->failed, 1); ALLOC(h->all_walkers, nw);
-    ALLOC(h->counters, (size_t)CNT_SLOTS);
+    ALLOC(h->counters, nw * CNT_SLOTS); ALLOC(h->total, (size_t)CNT_SLOTS + 1); ALLOC(h->nap, nw);
     ALLOC(h->logdet, 2 * nw); ALLOC(h->eloc, nw); ALLOC(h->drift, 2 * nw); ALLOC(h->dstats, 3);
     // refresh workspace: up to 16 GiB of FP64 work matrices per batch (about
     // 10000 walkers at 432 sites, so one launch pair covers even a refresh of
@@ -545,6 +578,15 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     for (size_t s = 0; s < ns; ++s) {
         off[s + 1] = off[s] + (int)adj[s].size();
         lst.insert(lst.end(), adj[s].begin(), adj[s].end());
+    }
+    std::vector<unsigned char> table(bond_table_bytes(h->ns, h->nb), 0);
+    {
+        uint32_t* tb = reinterpret_cast<uint32_t*>(table.data());
+        uint16_t* to = reinterpret_cast<uint16_t*>(tb + h->nb);
+        uint16_t* tn = to + ns + 1;
+        for (int b = 0; b < h->nb; ++b) tb[b] = (uint32_t)hb[b].x | ((uint32_t)hb[b].y << 16);
+        for (size_t s = 0; s <= ns; ++s) to[s] = (uint16_t)off[s];
+        for (size_t q = 0; q < lst.size(); ++q) tn[q] = (uint16_t)lst[q];
     }
     // U of the refresh (column-major) and its row-major copy.  Complex
     // orbitals (interleaved ns x N): the 2 ns x 2 N real form.
@@ -578,6 +620,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     if (up(h->bonds, hb.data(), hb.size() * sizeof(int2)) != hipSuccess ||
         up(h->nbr_off, off.data(), off.size() * sizeof(int)) != hipSuccess ||
         (lst.size() && up(h->nbr, lst.data(), lst.size() * sizeof(int)) != hipSuccess) ||
+        up(h->table, table.data(), table.size()) != hipSuccess ||
         up(h->Uup, ucu.data(), ucu.size() * sizeof(double)) != hipSuccess ||
         up(h->Udn, ucd.data(), ucd.size() * sizeof(double)) != hipSuccess ||
         (h->cplx && up(h->Ucup, d->u_up, 2 * ns * h->nup * sizeof(double)) != hipSuccess) ||
@@ -718,8 +761,7 @@ hipError_t enqueue_rounds(kvmc_handle* h, const SweepArgs& a, int threads, size_
                           hipStream_t s) {
     const int fb = (h->nw + 255) / 256;
     hipLaunchKernelGGL(k_set_stop, dim3(fb), dim3(256), 0, s, h->sweeps, h->stop, h->tbase, (long long)nsweeps,
-                       h->nw);
-    hipLaunchKernelGGL(k_fill_ull, dim3(1), dim3(64), 0, s, h->counters, 0ull, (int)CNT_SLOTS);
+                       h->nw, h->counters, h->total);
     hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, s, h->failed, INT_MAX, 1);
     hipError_t ce = hipGetLastError();
     for (int r = 0; r < kGraphRounds && ce == hipSuccess; ++r) {
@@ -788,7 +830,10 @@ int sweep_tail(kvmc_handle* h, const SweepArgs& a, int threads, size_t lds, bool
     if (outcomes && hipMemcpyAsync(outcomes, d_out, tape_n, hipMemcpyDeviceToHost, s) != hipSuccess)
         return fail(KVMC_ERR_HIP, "outcome copy failed");
     unsigned long long cnt[CNT_SLOTS] = {};
-    if (hipMemcpyAsync(cnt, h->counters, sizeof(cnt), hipMemcpyDeviceToHost, s) != hipSuccess ||
+    hipLaunchKernelGGL(k_sum_counters, dim3(std::min(8, (h->nw + 31) / 32)), dim3(256), 0, s, h->counters, h->total,
+                       h->nw);
+    HIP_TRY(hipGetLastError());
+    if (hipMemcpyAsync(cnt, h->total, sizeof(cnt), hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess)
         return fail(KVMC_ERR_HIP, "counter copy failed");
     if (counters) {
@@ -851,9 +896,8 @@ int sweep_staged(kvmc_handle* h, int64_t nsweeps, const double* tape_u, const in
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL(k_set_stop, dim3((h->nw + 255) / 256), dim3(256), 0, s,
-                           h->sweeps, h->stop, h->tbase, (long long)nsweeps, h->nw);
-        if (hipMemsetAsync(h->counters, 0, sizeof(unsigned long long) * CNT_SLOTS, s) != hipSuccess)
-            return fail(KVMC_ERR_HIP, "counter reset failed");
+                           h->sweeps, h->stop, h->tbase, (long long)nsweeps, h->nw, h->counters, h->total);
+        HIP_TRY(hipGetLastError());
     }
     return sweep_tail(h, a, threads, lds, finished, launches, outcomes, d_out, tape_n, counters);
 }
@@ -1037,7 +1081,7 @@ static ElocArgs eloc_args(kvmc_handle* h) {
     e.ns = h->ns; e.nup = h->nup; e.ndn = h->ndn; e.nb = h->nb;
     e.bonds = h->bonds; e.kup = h->kup; e.kdn = h->kdn; e.W = h->W; e.slot = h->slot; e.A = h->A; e.Bm = h->Bm;
     e.npend = h->npend; e.delay = h->delay; e.nmax = h->nmax; e.nw = h->nw;
-    e.eloc = h->eloc; e.eloc_im = h->eloc_im; e.counters = h->counters;
+    e.eloc = h->eloc; e.eloc_im = h->eloc_im; e.nap = h->nap;
     e.nparams = h->nparams; e.Qup = h->Qup; e.Qdn = h->Qdn; e.O = h->O;
     return e;
 }
@@ -1047,16 +1091,17 @@ int kvmc_measure(kvmc_handle* h, double* eloc, double* sum, int64_t* n_ap) {
     if (!h) return fail(KVMC_ERR_INVALID, "null handle");
     if (!h->ready) return fail(KVMC_ERR_NOT_READY, "configurations not set");
     hipStream_t s = h->stream;
-    HIP_TRY(hipMemsetAsync(h->counters + CNT_NAP, 0, sizeof(unsigned long long), s));
     prof_begin(h);
     HIP_TRY(do_eloc(h, eloc_args(h), s));
     prof_end(h);
+    hipLaunchKernelGGL(k_sum_nap, dim3(1), dim3(1024), 0, s, h->nap, h->total + CNT_SLOTS, h->nw);
+    HIP_TRY(hipGetLastError());
     std::vector<double> tmp;
     double* dst = eloc;
     if (!dst && sum) { tmp.resize(h->nw); dst = tmp.data(); }
     if (dst) HIP_TRY(hipMemcpyAsync(dst, h->eloc, sizeof(double) * h->nw, hipMemcpyDeviceToHost, s));
     unsigned long long nap = 0;
-    HIP_TRY(hipMemcpyAsync(&nap, h->counters + CNT_NAP, sizeof(nap), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(&nap, h->total + CNT_SLOTS, sizeof(nap), hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     h->prof.measure_ms += prof_elapsed(h);
     h->prof.measure_launches += h->profiling;

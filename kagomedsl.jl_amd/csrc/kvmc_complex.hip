@@ -4,11 +4,14 @@
 // 181-182, 290): W in complex float (FP32 form) or complex double (FP64).
 // The ratio's modulus squared, the delayed terms and the local energy are
 // the complex counterparts of the real kernels.  gfx950 only.
-#include "kvmc_kernels.hpp"
+#include "kvmc_sweep_res.hpp"
 
 namespace kvmc {
 
 hipError_t launch_sweep_c(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
+    // small clusters: W in LDS, one wavefront per walker
+    if (sweep_resident(w_elem_bytes(prec, 1), a.ns, a.nup, a.ndn) && sweep_w1_fits(a.ns, a.nup, a.ndn))
+        return prec == 0 ? launch_w1<cf64>(a, nw, s) : launch_w1<cf32>(a, nw, s);
     if (sweep_ib_supported(prec, 1, a.ns, a.nup, a.ndn, a.delay, a.nb)) return launch_sweep_ib(prec, 1, a, nw, s);
     // 16-byte vectors: two complex floats or one complex double
     if (prec == 0) return launch_sweep_v<cf64, 1>(a, nw, threads, lds, s);

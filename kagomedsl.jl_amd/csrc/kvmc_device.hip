@@ -1,6 +1,6 @@
 // Launchers of the sampler kernels (kvmc_kernels.hpp) for real orbitals:
 // W in float (FP32 form) or double (FP64 form).  gfx950 only.
-#include "kvmc_kernels.hpp"
+#include "kvmc_sweep_res.hpp"
 
 namespace kvmc {
 
@@ -15,6 +15,9 @@ size_t sweep_lds_bytes(size_t esize, int ns, int nup, int ndn, int delay, int nb
 }
 
 hipError_t launch_sweep(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
+    // small clusters: W in LDS, one wavefront per walker
+    if (sweep_resident(w_elem_bytes(prec, 0), a.ns, a.nup, a.ndn) && sweep_w1_fits(a.ns, a.nup, a.ndn))
+        return prec == 0 ? launch_w1<double>(a, nw, s) : launch_w1<float>(a, nw, s);
     // W streamed from HBM with columns of at most 256 rows and pending terms:
     // pending rows kept implicit (no row reads at an accept)
     if (sweep_ib_supported(prec, 0, a.ns, a.nup, a.ndn, a.delay, a.nb)) return launch_sweep_ib(prec, 0, a, nw, s);

@@ -12,9 +12,10 @@ enum : int { OUT_PRE_REJECT = 0, OUT_NO_MOVE = 1, OUT_REJECT = 2, OUT_ACCEPT = 3
 enum : int { KERNEL_REFERENCE = 0, KERNEL_UNBIASED = 1 };
 enum : int { POLICY_REFERENCE = 0, POLICY_EVERY_K = 1, POLICY_AT_END = 2 };
 
-// Device-wide counters (u64 slots).
-enum : int { CNT_MOVES = 0, CNT_ACCEPTED = 1, CNT_FLUSHES = 2, CNT_SWEEPS = 3, CNT_NAP = 4,
-             CNT_PAUSES = 5, CNT_SLOTS = 8 };
+// Counters of a sweep call (u64 slots), kept per walker and summed at its
+// end: with one set for the device, five atomics per walker on one cache line
+// took 174 of the 270 us of sweep kernels at 4096 walkers of 48 sites.
+enum : int { CNT_MOVES = 0, CNT_ACCEPTED = 1, CNT_FLUSHES = 2, CNT_SWEEPS = 3, CNT_PAUSES = 4, CNT_SLOTS = 8 };
 
 // Largest number of pending rank-1 updates kept per spin before a flush.
 constexpr int kMaxDelay = 16;
@@ -108,12 +109,20 @@ __host__ __device__ inline void sweep_draws(uint64_t seed, uint32_t walker, int6
     *bond = (int)(((uint64_t)x[2] * (uint64_t)(uint32_t)nb) >> 32);
 }
 
+// The bond tables as the sweep kernels keep them in LDS, one blob of whole
+// 16-byte vectors: nb packed site pairs (uint32), ns + 1 offsets and at most
+// 2 nb bond ids (uint16).
+__host__ __device__ inline size_t bond_table_bytes(int ns, int nb) {
+    return ((size_t)nb * sizeof(uint32_t) + (size_t)(ns + 1 + 2 * nb) * sizeof(uint16_t) + 15) / 16 * 16;
+}
+
 // Arguments of the sweep kernel.  Every pointer is device memory.
 struct SweepArgs {
     int ns, nup, ndn, nb, nocc;     // nocc = min(nup, ndn)
     const int2* bonds;              // nb pairs, 0-based
     const int* nbr_off;             // ns+1 offsets into nbr
     const int* nbr;                 // bond ids touching each site
+    const void* table;              // the three packed: bond_table_bytes
     int* kup;                       // [nw][ns] labels 1-based, 0 empty
     int* kdn;
     void* W;                        // [nw][w_stride] empty-site rows, column-major per spin
@@ -130,7 +139,7 @@ struct SweepArgs {
     int* acc_since;                 // [nw] accepted moves since last refresh
     int* refresh_list;              // walkers paused for a refresh
     int* refresh_count;
-    unsigned long long* counters;   // CNT_*
+    unsigned long long* counters;   // [nw][CNT_SLOTS]
     uint64_t seed;
     const double* tape_u;           // [nw][tape_len] or null
     const int* tape_bond;
@@ -196,7 +205,7 @@ struct ElocArgs {
     int nw;
     double* eloc;                   // [nw]
     double* eloc_im;                // [nw] imaginary part (complex W only; may be null)
-    unsigned long long* counters;   // CNT_NAP accumulates antiparallel counts
+    int* nap;                       // [nw] antiparallel bonds
     // log-derivatives: Q_k = dU_k U^H (ns x ns row-major per parameter and
     // spin; complex interleaved for complex W)
     int nparams;

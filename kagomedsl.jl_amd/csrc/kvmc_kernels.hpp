@@ -271,6 +271,50 @@ __device__ __forceinline__ int z_delta(const uint32_t* bonds, const uint16_t* nb
     return flip - 2 * ap;
 }
 
+// The change of Z (z_delta) when the electrons on the antiparallel pair
+// (i, j) are exchanged, one bond per lane; uniform result.
+__device__ __forceinline__ int z_delta_wave(const uint32_t* bonds, const uint16_t* nbr_off, const uint16_t* nbr,
+                                            const int16_t* s_kup, const int16_t* s_kdn, int i, int j, int lane) {
+    int dz = 0;
+#pragma unroll
+    for (int side = 0; side < 2; ++side) {
+        const int x = side ? j : i, other = side ? i : j;
+        const int p1 = nbr_off[x + 1];
+        for (int p0 = nbr_off[x]; p0 < p1; p0 += 64) {
+            bool flip = false, ap = false;
+            if (p0 + lane < p1) {
+                const uint32_t bp = bonds[nbr[p0 + lane]];
+                const int bx = (int)(bp & 0xffffu), by = (int)(bp >> 16);
+                const int y = bx == x ? by : bx;
+                flip = bx != by && y != other;
+                ap = flip && ((s_kup[bx] != 0 && s_kdn[by] != 0) || (s_kup[by] != 0 && s_kdn[bx] != 0));
+            }
+            dz += __popcll(__ballot(flip)) - 2 * __popcll(__ballot(ap));
+        }
+    }
+    return dz;
+}
+
+// The same value, recomputed from here on instead of kept.
+__device__ __forceinline__ int opaque_v(int x) { asm volatile("" : "+v"(x)); return x; }
+__device__ __forceinline__ int opaque_s(int x) { return __builtin_amdgcn_readfirstlane(opaque_v(x)); }
+
+// The kernel's arguments, loaded where they are used: those of the draws and
+// of the launch's exit are not held in scalar registers through the loop.
+typedef const __attribute__((address_space(4))) SweepArgs LateArgs;
+__device__ __forceinline__ LateArgs* late_args() {
+    unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return (LateArgs*)p;
+}
+
+// The wavefront reads from LDS what its own lanes wrote.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ inline double block_sum_double(double v, double* red) {
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     const int wave = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
@@ -509,12 +553,12 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3))) k
         if (pause || (a.policy == POLICY_AT_END && acc_since >= a.refresh_k)) {
             int slot = atomicAdd(a.refresh_count, 1);
             a.refresh_list[slot] = w;
-            atomicAdd(&a.counters[CNT_PAUSES], 1ull);
+            a.counters[(size_t)w * CNT_SLOTS + CNT_PAUSES] += 1ull;
         }
-        atomicAdd(&a.counters[CNT_MOVES], n_moves);
-        atomicAdd(&a.counters[CNT_ACCEPTED], n_acc);
-        atomicAdd(&a.counters[CNT_FLUSHES], n_flush);
-        atomicAdd(&a.counters[CNT_SWEEPS], n_sweeps);
+        a.counters[(size_t)w * CNT_SLOTS + CNT_MOVES] += n_moves;
+        a.counters[(size_t)w * CNT_SLOTS + CNT_ACCEPTED] += n_acc;
+        a.counters[(size_t)w * CNT_SLOTS + CNT_FLUSHES] += n_flush;
+        a.counters[(size_t)w * CNT_SLOTS + CNT_SWEEPS] += n_sweeps;
     }
 }
 
@@ -703,7 +747,7 @@ __global__ void __launch_bounds__(256) k_eloc(ElocArgs a) {
     if (lane == 0) {
         a.eloc[w] = v;
         if (is_cplx<T>::value && a.eloc_im) a.eloc_im[w] = offi;
-        atomicAdd(&a.counters[CNT_NAP], nap);
+        a.nap[w] = (int)nap;
     }
 }
 
@@ -807,7 +851,7 @@ __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
     if (t0 == 0) {
         a.eloc[w] = v;
         if (is_cplx<T>::value && a.eloc_im) a.eloc_im[w] = vi;
-        atomicAdd(&a.counters[CNT_NAP], (unsigned long long)napt);
+        a.nap[w] = (int)napt;
     }
 }
 

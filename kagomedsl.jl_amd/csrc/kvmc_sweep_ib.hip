@@ -116,26 +116,6 @@ __device__ __forceinline__ float xor4(float v) { return __shfl_xor(v, 4, 64); }
 __device__ __forceinline__ double xor4(double v) { return __shfl_xor(v, 4, 64); }
 __device__ __forceinline__ cf64 xor4(cf64 v) { return cf64(__shfl_xor(v.re, 4, 64), __shfl_xor(v.im, 4, 64)); }
 
-// The same value, recomputed from here on instead of kept.
-__device__ __forceinline__ int opaque_v(int x) { asm volatile("" : "+v"(x)); return x; }
-__device__ __forceinline__ int opaque_s(int x) { return __builtin_amdgcn_readfirstlane(opaque_v(x)); }
-
-// The kernel's arguments, loaded where they are used: those of the draws and
-// of the launch's exit are not held in scalar registers through the loop.
-typedef const __attribute__((address_space(4))) SweepArgs LateArgs;
-__device__ __forceinline__ LateArgs* late_args() {
-    unsigned long long p = (unsigned long long)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return (LateArgs*)p;
-}
-
-// The wavefront reads from LDS what its own lanes wrote.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 __device__ __forceinline__ float ib_mac(float v, float a, float b) { return v + a * b; }
 __device__ __forceinline__ double ib_mac(double v, double a, double b) { return v + a * b; }
 __device__ __forceinline__ cf64 ib_mac(cf64 v, cf64 a, cf64 b) {
@@ -261,30 +241,6 @@ __device__ __forceinline__ void apply_ib(T* __restrict__ W0, const T* __restrict
             }
         }
     }
-}
-
-// The change of Z (z_delta) when the electrons on the antiparallel pair
-// (i, j) are exchanged, one bond per lane; uniform result.
-__device__ __forceinline__ int z_delta_wave(const uint32_t* bonds, const uint16_t* nbr_off, const uint16_t* nbr,
-                                            const int16_t* s_kup, const int16_t* s_kdn, int i, int j, int lane) {
-    int dz = 0;
-#pragma unroll
-    for (int side = 0; side < 2; ++side) {
-        const int x = side ? j : i, other = side ? i : j;
-        const int p1 = nbr_off[x + 1];
-        for (int p0 = nbr_off[x]; p0 < p1; p0 += 64) {
-            bool flip = false, ap = false;
-            if (p0 + lane < p1) {
-                const uint32_t bp = bonds[nbr[p0 + lane]];
-                const int bx = (int)(bp & 0xffffu), by = (int)(bp >> 16);
-                const int y = bx == x ? by : bx;
-                flip = bx != by && y != other;
-                ap = flip && ((s_kup[bx] != 0 && s_kdn[by] != 0) || (s_kup[by] != 0 && s_kdn[bx] != 0));
-            }
-            dz += __popcll(__ballot(flip)) - 2 * __popcll(__ballot(ap));
-        }
-    }
-    return dz;
 }
 
 template <typename T, int DMAX, int M, int UNR, bool EX>
@@ -695,12 +651,12 @@ k_sweep_ib(SweepArgs a) {
         if (pause || (k->policy == POLICY_AT_END && acc_since >= k->refresh_k)) {
             const int s = atomicAdd(k->refresh_count, 1);
             k->refresh_list[s] = w;
-            atomicAdd(&k->counters[CNT_PAUSES], 1ull);
+            k->counters[(size_t)w * CNT_SLOTS + CNT_PAUSES] += 1ull;
         }
-        atomicAdd(&k->counters[CNT_MOVES], n_moves);
-        atomicAdd(&k->counters[CNT_ACCEPTED], n_acc);
-        atomicAdd(&k->counters[CNT_FLUSHES], n_flush);
-        atomicAdd(&k->counters[CNT_SWEEPS], (unsigned long long)(sweeps - sweeps0));
+        k->counters[(size_t)w * CNT_SLOTS + CNT_MOVES] += n_moves;
+        k->counters[(size_t)w * CNT_SLOTS + CNT_ACCEPTED] += n_acc;
+        k->counters[(size_t)w * CNT_SLOTS + CNT_FLUSHES] += n_flush;
+        k->counters[(size_t)w * CNT_SLOTS + CNT_SWEEPS] += (unsigned long long)(sweeps - sweeps0);
     }
 }
 
