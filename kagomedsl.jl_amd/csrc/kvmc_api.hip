@@ -105,21 +105,51 @@ void random_config(uint64_t seed, uint32_t walker, uint32_t attempt, int ns, int
     for (int b = 0; b < ndn; ++b) kdn[perm[nup + b]] = b + 1;
 }
 
-// Start of a sweep call: stop counts, the walkers' counters and their sums cleared.
+// What a call brings back to the host, in pinned memory that the kernels
+// write: a copy of a few bytes from device memory costs a kernel of its own.
+struct HostBlock {
+    unsigned long long total[CNT_SLOTS];   // counters of the sweep call so far, summed over walkers
+    unsigned long long nap;                // antiparallel bonds, summed over walkers
+    int count;                             // walkers the last sweep launch listed for a refresh
+    int failed;                            // smallest walker with a singular tildeU, INT_MAX: none
+};
+
+// Start of a sweep call: stop counts; counters, refresh list and failure cleared.
 __global__ void k_set_stop(const long long* sweeps, long long* stop, long long* base, long long nsweeps, int nw,
-                           unsigned long long* counters, unsigned long long* total) {
+                           unsigned long long* counters, int* rcount, int* failed) {
     int w = blockIdx.x * blockDim.x + threadIdx.x;
     if (w < nw) {
         base[w] = sweeps[w];
         stop[w] = sweeps[w] + nsweeps;
         for (int q = 0; q < CNT_SLOTS; ++q) counters[(size_t)w * CNT_SLOTS + q] = 0;
     }
-    if (w < CNT_SLOTS) total[w] = 0;
+    if (w == 0) {
+        *rcount = 0;
+        *failed = INT_MAX;
+    }
 }
 
-// total[slot] += sum over walkers of counters[walker][slot]; threads take the
-// slots in turn (blockDim a multiple of CNT_SLOTS).
-__global__ void __launch_bounds__(256) k_sum_counters(const unsigned long long* counters, unsigned long long* total, int nw) {
+// True in every thread of the last block of the grid to arrive, whose thread
+// 0 has reset the ticket; the other blocks' atomics have been done by then.
+__device__ bool last_block(int* ticket) {
+    __shared__ int last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        last = atomicAdd(ticket, 1) == (int)gridDim.x - 1;
+        if (last) *ticket = 0;
+    }
+    __syncthreads();
+    __threadfence();
+    return last != 0;
+}
+
+// End of a sweep launch: the counters summed over walkers, the number of
+// walkers listed for a refresh and the failure to the host; the list is
+// cleared for the next launch.  `total` is zero between calls.  256 threads,
+// which take the slots in turn.
+__global__ void __launch_bounds__(256) k_collect(const unsigned long long* counters, int nw, unsigned long long* total,
+                                                 int* ticket, int* rcount, const int* failed, HostBlock* out) {
     __shared__ unsigned long long part[256];
     const int t = (int)threadIdx.x;
     const size_t n = (size_t)nw * CNT_SLOTS, step = (size_t)gridDim.x * 256;
@@ -131,21 +161,53 @@ __global__ void __launch_bounds__(256) k_sum_counters(const unsigned long long* 
         for (int q = t + CNT_SLOTS; q < 256; q += CNT_SLOTS) v += part[q];
         atomicAdd(&total[t], v);
     }
+    if (!last_block(ticket)) return;
+    if (t < CNT_SLOTS) out->total[t] = atomicExch(&total[t], 0ull);
+    if (t == 0) {
+        out->count = *rcount;
+        out->failed = *failed;
+        *rcount = 0;
+    }
 }
 
-// *total = sum of nap over the walkers (one block).
-__global__ void __launch_bounds__(1024) k_sum_nap(const int* nap, unsigned long long* total, int nw) {
-    __shared__ unsigned long long part[16];
+// End of a measurement: the local energies (and their imaginary parts) and the
+// sum of nap to the host.
+__global__ void __launch_bounds__(256) k_collect_eloc(const double* eloc, const double* eloc_im, const int* nap, int nw,
+                                                      unsigned long long* total, int* ticket, double* he, HostBlock* out) {
+    __shared__ unsigned long long part[4];
     const int t = (int)threadIdx.x;
     unsigned long long v = 0;
-    for (int w = t; w < nw; w += 1024) v += (unsigned long long)nap[w];
+    for (int w = (int)blockIdx.x * 256 + t; w < nw; w += (int)gridDim.x * 256) {
+        he[w] = eloc[w];
+        if (eloc_im) he[(size_t)nw + w] = eloc_im[w];
+        v += (unsigned long long)nap[w];
+    }
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if (t % 64 == 0) part[t / 64] = v;
     __syncthreads();
-    if (t == 0) {
-        for (int q = 1; q < 16; ++q) v += part[q];
-        *total = v;
+    if (t == 0) atomicAdd(total, part[0] + part[1] + part[2] + part[3]);
+    if (!last_block(ticket)) return;
+    if (t == 0) out->nap = atomicExch(total, 0ull);
+}
+
+// The checks of validate_configs, a workgroup per walker: the smallest walker
+// that fails one (its message is made on the host).  seen: 2 (nmax + 1) ints.
+__global__ void __launch_bounds__(64) k_validate(const int* ku, const int* kd, int ns, int nup, int ndn, int nmax,
+                                                 int* bad) {
+    extern __shared__ int seen[];
+    const int w = (int)blockIdx.x, t = (int)threadIdx.x;
+    for (int q = t; q < 2 * (nmax + 1); q += 64) seen[q] = 0;
+    __syncthreads();
+    bool fail = false;
+    for (int s = t; s < ns; s += 64) {
+        const int lu = ku[(size_t)w * ns + s], ld = kd[(size_t)w * ns + s];
+        if ((lu != 0) == (ld != 0) || lu < 0 || lu > nup || ld < 0 || ld > ndn) fail = true;
+        else if (lu) fail |= atomicAdd(&seen[lu], 1) != 0;
+        else fail |= atomicAdd(&seen[nmax + 1 + ld], 1) != 0;
     }
+    __syncthreads();
+    for (int l = 1 + t; l <= nmax; l += 64) fail |= (l <= nup && seen[l] == 0) || (l <= ndn && seen[nmax + 1 + l] == 0);
+    if (__ballot(fail) && t == 0) atomicMin(bad, w);
 }
 
 __global__ void k_fill_ll(long long* p, long long v, int n) {
@@ -245,7 +307,11 @@ struct kvmc_handle {
     int* failed = nullptr;
     int* all_walkers = nullptr;
     unsigned long long* counters = nullptr;   // [nw][CNT_SLOTS] of the current sweep call
-    unsigned long long* total = nullptr;      // [CNT_SLOTS] their sums, then one slot for the sum of nap
+    unsigned long long* total = nullptr;      // [CNT_SLOTS + 1] their sums and that of nap while a kernel forms them
+    int* ticket = nullptr;                    // blocks done (last_block)
+    HostBlock* host = nullptr;                // pinned, written by kernels
+    double* host_e = nullptr;                 // pinned [2 nw]: energies (re, im), log-determinants
+    double* host_o = nullptr;                 // pinned: log-derivatives
     int* nap = nullptr;                       // [nw] antiparallel bonds of the last measurement
     double* logdet = nullptr;
     double* eloc = nullptr;
@@ -254,6 +320,7 @@ struct kvmc_handle {
     bool track_drift = false;       // drift pass before every policy refresh
     double* ws = nullptr;
     int ws_jobs = 0;
+    size_t ws_bytes = 0;
     int nparams = 0;
     double* Qup = nullptr;
     double* Qdn = nullptr;
@@ -284,10 +351,12 @@ void free_all(kvmc_handle* h) {
     void* ptrs[] = {h->bonds, h->nbr_off, h->nbr, h->table, h->Uup, h->Udn, h->UTup, h->UTdn, h->Ucup, h->Ucdn, h->kRup,
                     h->kRdn, h->eloc_im, h->kup, h->kdn, h->W, h->slot, h->A,
                     h->Bm, h->npend, h->pterm, h->zmu, h->acc_since, h->status, h->stiff, h->sweeps, h->stop,
-                    h->tbase, h->rlist, h->rcount, h->failed, h->all_walkers, h->counters, h->total, h->nap,
+                    h->tbase, h->rlist, h->rcount, h->failed, h->all_walkers, h->counters, h->total, h->ticket, h->nap,
                     h->logdet, h->eloc, h->drift, h->dstats, h->ws, h->Qup, h->Qdn, h->O};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    for (void* p : {(void*)h->host, (void*)h->host_e, (void*)h->host_o})
+        if (p) (void)hipHostFree(p);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
     if (h->gexec) (void)hipGraphExecDestroy(h->gexec);
@@ -316,7 +385,7 @@ SweepArgs sweep_args(kvmc_handle* h) {
     a.bonds = h->bonds; a.nbr_off = h->nbr_off; a.nbr = h->nbr; a.table = h->table;
     a.kup = h->kup; a.kdn = h->kdn; a.W = h->W; a.slot = h->slot; a.A = h->A; a.Bm = h->Bm;
     a.npend = h->npend; a.delay = h->delay; a.nmax = h->nmax;
-    a.pterm = h->pterm; a.stiff = h->stiff;
+    a.pterm = h->pterm; a.stiff = h->stiff; a.failed = h->failed;
     a.sweeps = h->sweeps; a.stop = h->stop; a.tape_base = h->tbase;
     a.zmu = h->zmu; a.acc_since = h->acc_since;
     a.refresh_list = h->rlist; a.refresh_count = h->rcount;
@@ -325,8 +394,15 @@ SweepArgs sweep_args(kvmc_handle* h) {
     return a;
 }
 
-// Refreshes the walkers listed in d_list[0..count) (device array).  When
-// write_w is 0 only the drift against the current W is measured.
+// A singular refresh that the last k_collect or refresh_list reported.
+int check_failed(kvmc_handle* h) {
+    const int failed = h->host->failed;
+    if (failed == INT_MAX) return KVMC_OK;
+    h->failed_walker = failed;
+    return fail(KVMC_ERR_SINGULAR, "tildeU is singular for walker " + std::to_string(failed) +
+                                       " (lu factorization failed)");
+}
+
 RefreshArgs refresh_args(const kvmc_handle* h, int write_w, double pivot_tol) {
     RefreshArgs r{};
     const int f = h->cplx ? 2 : 1;   // complex orbitals: the real form's doubled sizes
@@ -348,11 +424,14 @@ hipError_t prepare_refresh(kvmc_handle* h, hipStream_t s) {
     return e != hipSuccess ? e : launch_kappa_real_form(h->kdn, h->kRdn, h->ns, h->ndn, h->nw, s);
 }
 
+// Refreshes the walkers listed in d_list[0..count) (device array).  When
+// write_w is 0 only the drift against the current W is measured.
+// in_sweep: between two sweep launches of a call, whose start cleared the
+// failure and whose next k_collect reports it; else this call does both.
 int refresh_list(kvmc_handle* h, const int* d_list, int count, int write_w,
-                 double pivot_tol = 0.0, bool drift_first = false) {
+                 double pivot_tol = 0.0, bool drift_first = false, bool in_sweep = false) {
     if (count <= 0) return KVMC_OK;
-    static const int kNone = INT_MAX;
-    HIP_TRY(hipMemcpyAsync(h->failed, &kNone, sizeof(int), hipMemcpyHostToDevice, h->stream));
+    if (!in_sweep) hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, h->stream, h->failed, INT_MAX, 1);
     const int batch_walkers = std::max(1, h->ws_jobs / 2);
     const int fb = (count + 255) / 256;
     HIP_TRY(prepare_refresh(h, h->stream));
@@ -382,16 +461,14 @@ int refresh_list(kvmc_handle* h, const int* d_list, int count, int write_w,
         h->prof.refresh_launches += h->profiling;
     }
     prof_end(h);
-    int failed = INT_MAX;
-    HIP_TRY(hipMemcpyAsync(&failed, h->failed, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    if (in_sweep) {
+        h->prof.refresh_ms += prof_elapsed(h);
+        return KVMC_OK;
+    }
+    HIP_TRY(hipMemcpyAsync(&h->host->failed, h->failed, sizeof(int), hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     h->prof.refresh_ms += prof_elapsed(h);
-    if (failed != INT_MAX) {
-        h->failed_walker = failed;
-        return fail(KVMC_ERR_SINGULAR, "tildeU is singular for walker " + std::to_string(failed) +
-                                           " (lu factorization failed)");
-    }
-    return KVMC_OK;
+    return check_failed(h);
 }
 
 int refresh_all(kvmc_handle* h, int write_w) {
@@ -425,6 +502,40 @@ int upload_configs(kvmc_handle* h, const int32_t* ku, const int32_t* kd) {
     HIP_TRY(hipMemcpyAsync(h->kdn, kd, n * sizeof(int), hipMemcpyHostToDevice, h->stream));
     HIP_TRY(hipMemsetAsync(h->npend, 0, sizeof(int) * h->nw, h->stream));
     HIP_TRY(hipMemsetAsync(h->acc_since, 0, sizeof(int) * h->nw, h->stream));
+    return KVMC_OK;
+}
+
+// Uploads configurations after checking them.  They are checked on the device,
+// in the refresh workspace, so that wrong ones leave the handle as it is; the
+// host looks at the first wrong walker again for its message (and at all of
+// them where the workspace is too small).
+int upload_checked(kvmc_handle* h, const int32_t* ku, const int32_t* kd) {
+    const size_t n = (size_t)h->nw * h->ns;
+    if (h->ws_bytes < 2 * n * sizeof(int)) {
+        for (int w = 0; w < h->nw; ++w) {
+            int rc = validate_configs(h, ku + (size_t)w * h->ns, kd + (size_t)w * h->ns, w);
+            if (rc) return rc;
+        }
+        return upload_configs(h, ku, kd);
+    }
+    hipStream_t s = h->stream;
+    int* du = reinterpret_cast<int*>(h->ws);
+    int* dd = du + n;
+    HIP_TRY(hipMemcpyAsync(du, ku, n * sizeof(int), hipMemcpyHostToDevice, s));
+    HIP_TRY(hipMemcpyAsync(dd, kd, n * sizeof(int), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, s, h->failed, INT_MAX, 1);
+    hipLaunchKernelGGL(k_validate, dim3(h->nw), dim3(64), 2 * (h->nmax + 1) * sizeof(int), s, du, dd, h->ns, h->nup,
+                       h->ndn, h->nmax, h->failed);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipMemcpyAsync(&h->host->failed, h->failed, sizeof(int), hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
+    const int bad = h->host->failed;
+    if (bad != INT_MAX)
+        return validate_configs(h, ku + (size_t)bad * h->ns, kd + (size_t)bad * h->ns, bad);
+    HIP_TRY(hipMemcpyAsync(h->kup, du, n * sizeof(int), hipMemcpyDeviceToDevice, s));
+    HIP_TRY(hipMemcpyAsync(h->kdn, dd, n * sizeof(int), hipMemcpyDeviceToDevice, s));
+    HIP_TRY(hipMemsetAsync(h->npend, 0, sizeof(int) * h->nw, s));
+    HIP_TRY(hipMemsetAsync(h->acc_since, 0, sizeof(int) * h->nw, s));
     return KVMC_OK;
 }
 
@@ -553,6 +664,11 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
     ALLOC(h->sweeps, nw); ALLOC(h->stop, nw); ALLOC(h->tbase, nw);
     ALLOC(h->rlist, nw); ALLOC(h->rcount, 1); ALLOC(h->failed, 1); ALLOC(h->all_walkers, nw);
     ALLOC(h->counters, nw * CNT_SLOTS); ALLOC(h->total, (size_t)CNT_SLOTS + 1); ALLOC(h->nap, nw);
+    ALLOC(h->ticket, 1);
+    if (hipHostMalloc(reinterpret_cast<void**>(&h->host), sizeof(HostBlock), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&h->host_e), 2 * nw * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        free_all(h); delete h; return fail(KVMC_ERR_NOMEM, "hipHostMalloc of the result buffers failed");
+    }
     ALLOC(h->logdet, 2 * nw); ALLOC(h->eloc, nw); ALLOC(h->drift, 2 * nw); ALLOC(h->dstats, 3);
     // refresh workspace: up to 16 GiB of FP64 work matrices per batch (about
     // 10000 walkers at 432 sites, so one launch pair covers even a refresh of
@@ -564,6 +680,7 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
         h->ws_jobs = (int)(jobs & ~(size_t)1);
         if (h->ws_jobs < 2) h->ws_jobs = 2;
         ALLOC(h->ws, (size_t)h->ws_jobs * refresh_ws_doubles_per_job(cf * h->ns, cf * h->nmax));
+        h->ws_bytes = (size_t)h->ws_jobs * per_job;
     }
 #undef ALLOC
     // bonds (0-based) and site -> bond adjacency
@@ -634,6 +751,8 @@ int kvmc_create(const kvmc_desc* d, kvmc_handle** out) {
         hipMemsetAsync(h->acc_since, 0, nw * sizeof(int), h->stream) != hipSuccess ||
         hipMemsetAsync(h->logdet, 0, 2 * nw * sizeof(double), h->stream) != hipSuccess ||
         hipMemsetAsync(h->dstats, 0, 3 * sizeof(double), h->stream) != hipSuccess ||
+        hipMemsetAsync(h->total, 0, (CNT_SLOTS + 1) * sizeof(unsigned long long), h->stream) != hipSuccess ||
+        hipMemsetAsync(h->ticket, 0, sizeof(int), h->stream) != hipSuccess ||
         hipStreamSynchronize(h->stream) != hipSuccess) {
         free_all(h);
         delete h;
@@ -654,11 +773,7 @@ int kvmc_destroy(kvmc_handle* h) {
 int kvmc_set_configs(kvmc_handle* h, const int32_t* ku, const int32_t* kd) {
     g_err.clear();
     if (!h || !ku || !kd) return fail(KVMC_ERR_INVALID, "null argument");
-    for (int w = 0; w < h->nw; ++w) {
-        int rc = validate_configs(h, ku + (size_t)w * h->ns, kd + (size_t)w * h->ns, w);
-        if (rc) return rc;
-    }
-    int rc = upload_configs(h, ku, kd);
+    int rc = upload_checked(h, ku, kd);
     if (rc) return rc;
     h->failed_walker = -1;
     rc = refresh_all(h, 1);
@@ -753,6 +868,12 @@ int tape_check(const kvmc_handle* h, size_t tape_n, const double* tape_u, const 
     return KVMC_OK;
 }
 
+hipError_t enqueue_collect(kvmc_handle* h, hipStream_t s) {
+    hipLaunchKernelGGL(k_collect, dim3(std::min(16, (h->nw + 63) / 64)), dim3(256), 0, s, h->counters, h->nw, h->total,
+                       h->ticket, h->rcount, h->failed, h->host);
+    return hipGetLastError();
+}
+
 // Enqueues one captured sweep sequence of handle h on stream s: stop counts,
 // counter and flag resets (fill kernels, no memset nodes), then
 // kGraphRounds rounds of the sweep kernel, each but the last followed by
@@ -761,8 +882,7 @@ hipError_t enqueue_rounds(kvmc_handle* h, const SweepArgs& a, int threads, size_
                           hipStream_t s) {
     const int fb = (h->nw + 255) / 256;
     hipLaunchKernelGGL(k_set_stop, dim3(fb), dim3(256), 0, s, h->sweeps, h->stop, h->tbase, (long long)nsweeps,
-                       h->nw, h->counters, h->total);
-    hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, s, h->failed, INT_MAX, 1);
+                       h->nw, h->counters, h->rcount, h->failed);
     hipError_t ce = hipGetLastError();
     for (int r = 0; r < kGraphRounds && ce == hipSuccess; ++r) {
         hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, s, h->rcount, 0, 1);
@@ -779,25 +899,19 @@ hipError_t enqueue_rounds(kvmc_handle* h, const SweepArgs& a, int threads, size_
             ce = launch_refresh(h->prec, ra, s);
         }
     }
-    return ce;
+    return ce != hipSuccess ? ce : enqueue_collect(h, s);
 }
 
-// After a replay of enqueue_rounds: reports a singular refresh, refreshes
-// the walkers the last round paused; *finished when nothing is left to run.
+// After a replay of enqueue_rounds has completed: reports a singular refresh,
+// refreshes the walkers the last round paused; *finished when nothing is left
+// to run.
 int after_replay(kvmc_handle* h, bool* finished) {
-    hipStream_t s = h->stream;
-    int count = 0, failed = INT_MAX;
-    HIP_TRY(hipMemcpyAsync(&count, h->rcount, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(&failed, h->failed, sizeof(int), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (failed != INT_MAX) {
-        h->failed_walker = failed;
-        return fail(KVMC_ERR_SINGULAR, "tildeU is singular for walker " + std::to_string(failed) +
-                                           " (lu factorization failed)");
-    }
+    int rc = check_failed(h);
+    if (rc) return rc;
+    const int count = h->host->count;
     *finished = count == 0;
     if (count > 0) {
-        int rc = refresh_list(h, h->rlist, count, 1, 0.0, h->track_drift);
+        rc = refresh_list(h, h->rlist, count, 1, 0.0, h->track_drift);
         if (rc) return rc;
         *finished = h->policy == KVMC_REFRESH_AT_END;
     }
@@ -810,32 +924,29 @@ int sweep_tail(kvmc_handle* h, const SweepArgs& a, int threads, size_t lds, bool
                int8_t* outcomes, const signed char* d_out, size_t tape_n, kvmc_counters* counters) {
     hipStream_t s = h->stream;
     while (!finished) {
-        int count = 0;
-        if (hipMemsetAsync(h->rcount, 0, sizeof(int), s) != hipSuccess) return fail(KVMC_ERR_HIP, "hipMemsetAsync failed");
         prof_begin(h);
         hipError_t e = do_sweep(h, a, h->nw, threads, lds, s);
         if (e != hipSuccess) return fail(KVMC_ERR_HIP, std::string("sweep launch: ") + hipGetErrorString(e));
         prof_end(h);
         ++launches;
-        if (hipMemcpyAsync(&count, h->rcount, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
+        HIP_TRY(enqueue_collect(h, s));
+        if (hipStreamSynchronize(s) != hipSuccess)
             return fail(KVMC_ERR_HIP, std::string("sweep kernel: ") + hipGetErrorString(hipGetLastError()));
         h->prof.sweep_ms += prof_elapsed(h);
         h->prof.sweep_launches += h->profiling;
-        if (count == 0) break;
-        int rc = refresh_list(h, h->rlist, count, 1, 0.0, h->track_drift);
+        int rc = check_failed(h);
         if (rc) return rc;
-        if (h->policy == KVMC_REFRESH_AT_END) break;   // listed walkers had finished
+        const int count = h->host->count;
+        if (count == 0) break;
+        // AT_END: listed walkers had finished
+        finished = h->policy == KVMC_REFRESH_AT_END;
+        rc = refresh_list(h, h->rlist, count, 1, 0.0, h->track_drift, !finished);
+        if (rc) return rc;
     }
-    if (outcomes && hipMemcpyAsync(outcomes, d_out, tape_n, hipMemcpyDeviceToHost, s) != hipSuccess)
+    if (outcomes && (hipMemcpyAsync(outcomes, d_out, tape_n, hipMemcpyDeviceToHost, s) != hipSuccess ||
+                     hipStreamSynchronize(s) != hipSuccess))
         return fail(KVMC_ERR_HIP, "outcome copy failed");
-    unsigned long long cnt[CNT_SLOTS] = {};
-    hipLaunchKernelGGL(k_sum_counters, dim3(std::min(8, (h->nw + 31) / 32)), dim3(256), 0, s, h->counters, h->total,
-                       h->nw);
-    HIP_TRY(hipGetLastError());
-    if (hipMemcpyAsync(cnt, h->total, sizeof(cnt), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-        return fail(KVMC_ERR_HIP, "counter copy failed");
+    const unsigned long long* cnt = h->host->total;
     if (counters) {
         counters->sweeps = (int64_t)cnt[CNT_SWEEPS];
         counters->moves = (int64_t)cnt[CNT_MOVES];
@@ -891,12 +1002,13 @@ int sweep_staged(kvmc_handle* h, int64_t nsweeps, const double* tape_u, const in
             h->g_nsweeps = nsweeps;
         }
         HIP_TRY(hipGraphLaunch(h->gexec, s));
+        HIP_TRY(hipStreamSynchronize(s));
         launches += kGraphRounds;
         int rc = after_replay(h, &finished);
         if (rc) return rc;
     } else {
         hipLaunchKernelGGL(k_set_stop, dim3((h->nw + 255) / 256), dim3(256), 0, s,
-                           h->sweeps, h->stop, h->tbase, (long long)nsweeps, h->nw, h->counters, h->total);
+                           h->sweeps, h->stop, h->tbase, (long long)nsweeps, h->nw, h->counters, h->rcount, h->failed);
         HIP_TRY(hipGetLastError());
     }
     return sweep_tail(h, a, threads, lds, finished, launches, outcomes, d_out, tape_n, counters);
@@ -1086,6 +1198,16 @@ static ElocArgs eloc_args(kvmc_handle* h) {
     return e;
 }
 
+// The energies of the last eloc kernel and the sum of nap in host_e and host,
+// after the stream has finished.
+static int collect_eloc(kvmc_handle* h) {
+    hipLaunchKernelGGL(k_collect_eloc, dim3(std::min(64, (h->nw + 255) / 256)), dim3(256), 0, h->stream, h->eloc,
+                       h->cplx ? h->eloc_im : nullptr, h->nap, h->nw, h->total + CNT_SLOTS, h->ticket, h->host_e, h->host);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return KVMC_OK;
+}
+
 int kvmc_measure(kvmc_handle* h, double* eloc, double* sum, int64_t* n_ap) {
     g_err.clear();
     if (!h) return fail(KVMC_ERR_INVALID, "null handle");
@@ -1094,23 +1216,17 @@ int kvmc_measure(kvmc_handle* h, double* eloc, double* sum, int64_t* n_ap) {
     prof_begin(h);
     HIP_TRY(do_eloc(h, eloc_args(h), s));
     prof_end(h);
-    hipLaunchKernelGGL(k_sum_nap, dim3(1), dim3(1024), 0, s, h->nap, h->total + CNT_SLOTS, h->nw);
-    HIP_TRY(hipGetLastError());
-    std::vector<double> tmp;
-    double* dst = eloc;
-    if (!dst && sum) { tmp.resize(h->nw); dst = tmp.data(); }
-    if (dst) HIP_TRY(hipMemcpyAsync(dst, h->eloc, sizeof(double) * h->nw, hipMemcpyDeviceToHost, s));
-    unsigned long long nap = 0;
-    HIP_TRY(hipMemcpyAsync(&nap, h->total + CNT_SLOTS, sizeof(nap), hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    int rc = collect_eloc(h);
+    if (rc) return rc;
     h->prof.measure_ms += prof_elapsed(h);
     h->prof.measure_launches += h->profiling;
+    if (eloc) std::memcpy(eloc, h->host_e, sizeof(double) * h->nw);
     if (sum) {
         double acc = 0.0;
-        for (int w = 0; w < h->nw; ++w) acc += dst[w];
+        for (int w = 0; w < h->nw; ++w) acc += h->host_e[w];
         *sum = acc;
     }
-    if (n_ap) *n_ap = (int64_t)nap;
+    if (n_ap) *n_ap = (int64_t)h->host->nap;
     return KVMC_OK;
 }
 
@@ -1122,6 +1238,7 @@ int kvmc_set_orbital_derivs(kvmc_handle* h, int32_t nparams, const double* du_up
     if (h->Qup) { (void)hipFree(h->Qup); h->Qup = nullptr; }
     if (h->Qdn) { (void)hipFree(h->Qdn); h->Qdn = nullptr; }
     if (h->O) { (void)hipFree(h->O); h->O = nullptr; }
+    if (h->host_o) { (void)hipHostFree(h->host_o); h->host_o = nullptr; }
     h->nparams = 0;
     if (nparams == 0) return KVMC_OK;
     const size_t ns = h->ns;
@@ -1143,6 +1260,11 @@ int kvmc_set_orbital_derivs(kvmc_handle* h, int32_t nparams, const double* du_up
     HIP_TRY(hipMemcpyAsync(dU.p, du_dn, cw * nparams * ns * h->ndn * sizeof(double), hipMemcpyHostToDevice, s));
     HIP_TRY(q_build(h->cplx ? h->Ucdn : h->Udn, h->ndn, qd.p));
     HIP_TRY(hipStreamSynchronize(s));
+    if (hipHostMalloc(reinterpret_cast<void**>(&h->host_o), cw * nparams * h->nw * sizeof(double),
+                      hipHostMallocDefault) != hipSuccess) {
+        h->host_o = nullptr;
+        return fail(KVMC_ERR_NOMEM, "hipHostMalloc of the log-derivatives failed");
+    }
     h->Qup = qu.release();
     h->Qdn = qd.release();
     h->O = o.release();
@@ -1160,23 +1282,24 @@ int kvmc_measure_grad(kvmc_handle* h, double* eloc, double* o) {
     HIP_TRY(do_flush(h, a, h->nw, s));
     HIP_TRY(do_eloc(h, eloc_args(h), s));
     HIP_TRY(do_grad(h, eloc_args(h), s));
-    const size_t cw = h->cplx ? 2 : 1;
-    std::vector<double> re, im;
-    if (eloc && h->cplx) { re.resize(h->nw); im.resize(h->nw); }
-    if (eloc) HIP_TRY(hipMemcpyAsync(h->cplx ? re.data() : eloc, h->eloc, sizeof(double) * h->nw, hipMemcpyDeviceToHost, s));
-    if (eloc && h->cplx) HIP_TRY(hipMemcpyAsync(im.data(), h->eloc_im, sizeof(double) * h->nw, hipMemcpyDeviceToHost, s));
-    if (o) HIP_TRY(hipMemcpyAsync(o, h->O, cw * sizeof(double) * h->nw * h->nparams, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    if (eloc && h->cplx)
-        for (int w = 0; w < h->nw; ++w) { eloc[2 * w] = re[w]; eloc[2 * w + 1] = im[w]; }
+    const size_t cw = h->cplx ? 2 : 1, no = cw * h->nw * h->nparams;
+    if (o) HIP_TRY(hipMemcpyAsync(h->host_o, h->O, no * sizeof(double), hipMemcpyDeviceToHost, s));
+    int rc = collect_eloc(h);
+    if (rc) return rc;
+    if (o) std::memcpy(o, h->host_o, no * sizeof(double));
+    if (eloc)
+        for (int w = 0; w < h->nw; ++w) {
+            eloc[cw * w] = h->host_e[w];
+            if (h->cplx) eloc[2 * w + 1] = h->host_e[(size_t)h->nw + w];
+        }
     return KVMC_OK;
 }
 
 int kvmc_get_logdet(kvmc_handle* h, double* logdet) {
     g_err.clear();
     if (!h || !logdet) return fail(KVMC_ERR_INVALID, "null argument");
-    std::vector<double> two((size_t)2 * h->nw);
-    HIP_TRY(hipMemcpyAsync(two.data(), h->logdet, two.size() * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    const double* two = h->host_e;
+    HIP_TRY(hipMemcpyAsync(h->host_e, h->logdet, 2 * sizeof(double) * h->nw, hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     // complex orbitals: the real form's determinant is |det tildeU|^2
     const double f = h->cplx ? 0.5 : 1.0;

@@ -140,6 +140,7 @@ struct SweepArgs {
     int* refresh_list;              // walkers paused for a refresh
     int* refresh_count;
     unsigned long long* counters;   // [nw][CNT_SLOTS]
+    const int* failed;              // not INT_MAX after a singular refresh of this call: nothing is swept any more
     uint64_t seed;
     const double* tape_u;           // [nw][tape_len] or null
     const int* tape_bond;

@@ -377,7 +377,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3))) k
 
     long long sweeps = a.sweeps[w];
     const long long stop = a.stop[w];
-    if (sweeps >= stop) return;
+    if (sweeps >= stop || *a.failed != 0x7fffffff) return;
     int c = a.npend[w];
     int acc_since = a.acc_since[w];
 

@@ -286,7 +286,7 @@ k_sweep_ib(SweepArgs a) {
 
     long long sweeps = a.sweeps[w];
     const long long stop = a.stop[w];
-    if (sweeps >= stop) return;
+    if (sweeps >= stop || *a.failed != 0x7fffffff) return;
     int c = a.npend[w];
     int acc_since = a.acc_since[w];
     // FP64: a walker whose last refresh found a nearly singular tildeU (its W

@@ -113,7 +113,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     const long long stop = a.stop[w];
     int c = a.npend[w];
     int acc_since = a.acc_since[w];
-    if (sweeps >= stop) return;
+    if (sweeps >= stop || *a.failed != 0x7fffffff) return;
     {
         // labels and rows first, so that their loads are under way with W's
         const int* ku = a.kup + (size_t)w * ns;
