@@ -7,26 +7,23 @@
 // sites.  Row interchanges are implicit: phys[] maps the logical (pivoted)
 // row order onto physical rows, so no row of M ever moves.
 //
-// Two paths share the LU code (k_refresh_blocked, one 256-thread workgroup
-// per (walker, spin)):
-//
 // N <= 256: two kernels.
-//   k_refresh_blocked<FULL = false> factors tildeU alone: P tildeU = L1 U1,
-//   right-looking, panels of RB = 32 columns; the panel lives in registers
-//   (one row per thread) and one barrier per pivot column publishes each
-//   wavefront's best candidate row.  U12 = L11^-1 A12 and the trailing
-//   update run on FP64 MFMA (v_mfma_f64_16x16x4f64).  It saves L1, U1, the
-//   32x32 inverses of the diagonal blocks of L1 and U1 and the final row map.
+//   k_lu factors tildeU alone, P tildeU = L1 U1, panels of RB = 32 columns (see
+//   there).  It saves L1, U1, the inverses of their diagonal blocks and the
+//   final row map.
 //   k_refresh_solve then forms the empty-site rows of W: every wavefront
 //   holds 16 empty sites, i.e. their rows b of U transposed, as 16x16 MFMA
 //   accumulator tiles in registers, and solves y U1 = b and x L1 = y in place
 //   (block rows of the factors staged through LDS, shared by the four
 //   wavefronts).  W[s][phys[c]] = x[c]; occupied rows of W are unit rows.
 //
-// N > 256 (register tiles would not fit): one kernel, k_refresh_blocked<FULL
-// = true>, factors the tall matrix [tildeU ; U_empty] (rows >= N end as
-// L2 = U_empty U1^-1), solves X L1 = L2 panel by panel on MFMA and writes
-// W_empty = X P through LDS.
+// N > 256 (register tiles would not fit): one kernel of a 256-thread
+// workgroup per (walker, spin), k_refresh_blocked, right-looking: the panel in
+// registers (one row per thread and more), one barrier per pivot column to
+// publish each wavefront's best candidate row, U12 = L11^-1 A12 and the
+// trailing update on FP64 MFMA (v_mfma_f64_16x16x4f64).  It factors the tall
+// matrix [tildeU ; U_empty] (rows >= N end as L2 = U_empty U1^-1), solves
+// X L1 = L2 panel by panel and writes W_empty = X P through LDS.
 #include "kvmc_internal.hpp"
 
 #include <math.h>
@@ -47,7 +44,6 @@ constexpr int RB = 32;    // panel width
 constexpr int RT = 256;   // threads per workgroup
 constexpr int NWAVE = RT / 64;
 constexpr int LB = RB + 1;  // LDS row stride of 32-wide blocks
-constexpr int LU_WAVES = 3;  // waves per SIMD of the LU-only kernel
 constexpr int kStoreBlock = 8;   // sites per LDS block of the single kernel's W store
 
 __host__ __device__ inline int rup_i(int x, int m) { return (x + m - 1) / m * m; }
@@ -109,33 +105,6 @@ __device__ __attribute__((noinline)) void unit_lower_inverse(const double* L, do
     }
 }
 
-// 16 x 16 diagonal blocks at (off, off) of the same inverses, for the
-// two-kernel path, one block per wavefront: lanes 0..15 of wavefront `wv`
-// each hold one column.  Rows >= jb of the block are unit rows.
-__device__ __attribute__((noinline)) void unit_lower_inverse16(const double* L, double* Linv, int off, int jb, int wv) {
-    if ((int)threadIdx.x / 64 != wv) return;
-    const int j = (int)threadIdx.x & 15;
-    double x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        double v = (i == j) ? 1.0 : 0.0;
-        if (i > j && off + i < jb) {
-            double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-            for (int k = 0; k < i; k += 2) {
-                s0 += L[(off + i) * LB + off + k] * x[k];
-                if (k + 1 < i) s1 += L[(off + i) * LB + off + k + 1] * x[k + 1];
-            }
-            v = -(s0 + s1);
-        }
-        x[i] = v;
-    }
-    if ((threadIdx.x & 63) < 16) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) Linv[(off + i) * LB + off + j] = x[i];
-    }
-}
-
 __device__ __forceinline__ unsigned long long readlane64(unsigned long long k, int l) {
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)k, l);
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(k >> 32), l);
@@ -173,28 +142,6 @@ __device__ __attribute__((noinline)) void upper_inverse(const double* D, double*
     if (lane < RB) {
 #pragma unroll
         for (int i = 0; i < RB; ++i) Uinv[i * ld + j] = x[i];
-    }
-}
-
-__device__ __attribute__((noinline)) void upper_inverse16(const double* D, double* Uinv, int ld, int off, int wv) {
-    if ((int)threadIdx.x / 64 != wv) return;
-    const int lane = (int)threadIdx.x & 63;
-    const int j = lane & 15;
-    const double dinv = 1.0 / D[(off + j) * LB + off + j];
-    double x[16];
-#pragma unroll
-    for (int i = 15; i >= 0; --i) {
-        double s0 = (i == j) ? 1.0 : 0.0, s1 = 0.0;
-#pragma unroll
-        for (int k = i + 1; k < 16; k += 2) {
-            s0 -= D[(off + i) * LB + off + k] * x[k];
-            if (k + 1 < 16) s1 -= D[(off + i) * LB + off + k + 1] * x[k + 1];
-        }
-        x[i] = (s0 + s1) * readlane_f64(dinv, i);
-    }
-    if (lane < 16) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) Uinv[(off + i) * ld + off + j] = x[i];
     }
 }
 
@@ -240,8 +187,674 @@ __device__ __forceinline__ double rcp_f64(double x) {
     return fma(r, fma(-x, r, 1.0), r);
 }
 
-template <typename T, int RPT, bool FULL>
-__global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 2 : LU_WAVES))) k_refresh_blocked(RefreshArgs a) {
+// 16 x 16 diagonal blocks at (off, off) of the same inverses, for the
+// two-kernel path, one block per wavefront: lanes 0..15 of wavefront `wv`
+// each hold one column.  Rows >= jb of the block are unit rows.
+__device__ __attribute__((noinline)) void unit_lower_inverse16(const double* L, double* Linv, int off, int jb, int wv) {
+    if ((int)threadIdx.x / 64 != wv) return;
+    const int j = (int)threadIdx.x & 15;
+    double x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        double v = (i == j) ? 1.0 : 0.0;
+        if (i > j && off + i < jb) {
+            double s0 = 0.0, s1 = 0.0;
+#pragma unroll
+            for (int k = 0; k < i; k += 2) {
+                s0 += L[(off + i) * LB + off + k] * x[k];
+                if (k + 1 < i) s1 += L[(off + i) * LB + off + k + 1] * x[k + 1];
+            }
+            v = -(s0 + s1);
+        }
+        x[i] = v;
+    }
+    if ((threadIdx.x & 63) < 16) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Linv[(off + i) * LB + off + j] = x[i];
+    }
+}
+
+// Maximum of a 32-bit value over the wavefront, uniform result.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v) {
+    const uint32_t o = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+    return o > v ? o : v;
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = dpp_max_u32<0xB1>(v);
+    v = dpp_max_u32<0x4E>(v);
+    v = dpp_max_u32<0x141>(v);
+    v = dpp_max_u32<0x140>(v);
+    const uint32_t m0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), m1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    const uint32_t m2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), m3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    const uint32_t a = m0 > m1 ? m0 : m1, b = m2 > m3 ? m2 : m3;
+    return a > b ? a : b;
+}
+
+// Both 16x16 diagonal blocks of the inverse of the unit-lower block L, by the
+// calling wavefront: lanes 0..31 each hold one column in registers.  Rows >=
+// jb are unit rows.
+__device__ __forceinline__ void unit_lower_inverse16x2(const double* L, double* Linv, int jb, int lane) {
+    const int j = lane & 15, off = lane & 16;
+    const double* l = L + off * LB + off;
+    double x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        double v = (i == j) ? 1.0 : 0.0, s0 = 0.0, s1 = 0.0;
+#pragma unroll
+        for (int k = 0; k < i; k += 2) {
+            s0 += l[i * LB + k] * x[k];
+            if (k + 1 < i) s1 += l[i * LB + k + 1] * x[k + 1];
+        }
+        x[i] = (i > j && off + i < jb) ? -(s0 + s1) : v;
+    }
+    if (lane < 32) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Linv[(off + i) * LB + off + j] = x[i];
+    }
+}
+
+// The same of the upper-triangular block D (rows >= jb must be unit rows):
+// lane j of a block computes 1/D[j][j] once and the others read it through
+// readlane; entries below the diagonal come out zero.
+__device__ __forceinline__ void upper_inverse16x2(const double* D, double* Uinv, int ld, int lane) {
+    const int j = lane & 15, off = lane & 16;
+    const double* d = D + off * LB + off;
+    const double dinv = 1.0 / d[j * LB + j];
+    double x[16];
+#pragma unroll
+    for (int i = 15; i >= 0; --i) {
+        double s0 = (i == j) ? 1.0 : 0.0, s1 = 0.0;
+#pragma unroll
+        for (int k = i + 1; k < 16; k += 2) {
+            s0 -= d[i * LB + k] * x[k];
+            if (k + 1 < 16) s1 -= d[i * LB + k + 1] * x[k + 1];
+        }
+        const double r0 = readlane_f64(dinv, i), r1 = readlane_f64(dinv, 16 + i);
+        x[i] = (s0 + s1) * (off ? r1 : r0);
+    }
+    if (lane < 32) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Uinv[(off + i) * ld + off + j] = x[i];
+    }
+}
+
+// Pivoted LU of tildeU for N <= 32 NB: P tildeU = L1 U1, left-looking, panels
+// of RB = 32 columns, LUW wavefronts per (walker, spin).
+//
+// Wavefront 0 factors panel J alone, in two halves of 16 columns whose rows it
+// holds in registers (RPL a lane): a pivot search is two 32-bit maxima over
+// the wavefront, and the pivot row passes through LDS without a barrier.
+// Between the halves the first is applied to the second on MFMA, the rows
+// lying in LDS.  Meanwhile the other wavefronts take the columns of panel
+// J + 1, 16 at a time, from U through the panels before J, in MFMA
+// accumulators for all rows: U rows as L11_p^-1 times the block, whose result
+// is at once the operand of the rows below.  What is left for all is panel
+// J's own step on those columns.
+//
+// Bound: the chain of pivots, about 1700 cycles a column (key, maxima, LDS
+// round trip, reciprocal, update), and in the steps the reads of L, which lies
+// beyond L2 for the jobs in flight.  A panel in the registers of four
+// wavefronts, with a barrier and an LDS exchange a column, kept the matrix
+// cores waiting for it (64% of the time at N = 96, 42% at 216), and its
+// right-looking update read and wrote every trailing element once a panel.
+// Measured, LU and solve together: N = 96 881 -> 573 us (3037 matrices), 150
+// 1980 -> 1733 (3000), 216 3010 -> 2678 (2315), 54 109 -> 88 (about 1550).
+//
+// LUW = 3 above 128 columns (the two wavefronts beside the panel read the same
+// L tiles, and one alone is slower than the panel: 2918 against 2717 us at
+// N = 216), 2 up to 128 (585 against 620 at N = 96: more workgroups per CU)
+// and above 224 (three would need 102 more registers than they have).
+//
+// Every element sees its products in the order of the pivots, one fused
+// multiply-add each (the MFMA sums run in that order too), and U rows as
+// L11^-1 times the block, however the work is cut.
+template <int NB, int LUW>
+__global__ void __launch_bounds__(64 * LUW) __attribute__((amdgpu_waves_per_eu(NB > 7 ? 2 : NB > 4 ? 3 : 4))) k_lu(RefreshArgs a) {
+    constexpr int TH = 64 * LUW, RPL = (NB + 1) / 2, HB = RB / 2;
+    constexpr int UC = NB == 7 ? 4 : 8;                  // pivot row entries read ahead in a pivot step
+    constexpr int PD = NB > 7 ? 4 : 2;                   // row tiles whose L operands are under way
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int job = (int)blockIdx.x;
+    if (job >= a.njobs) return;
+    if (a.count_dev && job >= 2 * (*a.count_dev - a.walker_off)) return;
+    const int w = a.jobs[job >> 1];
+    const int spin = job & 1;
+    const int ns = a.ns, N = spin ? a.ndn : a.nup, nmax = a.nmax;
+    const int nrows = refresh_nrows(ns), ldm = refresh_ldm(nmax);
+    const int nc16 = rup_i(N, 16);                       // rows and columns that carry data
+    const double* __restrict__ UT = spin ? a.UTdn : a.UTup;   // ns x N row-major
+    const int* __restrict__ kap = (spin ? a.kdn : a.kup) + (size_t)w * ns;
+    double* M = a.ws + (size_t)job * refresh_ws_job(ns, nmax);
+    double* Lsave = M + (size_t)nrows * ldm;             // [npanel][RB][RB] inverses of L11
+    double* Usave = Lsave + (size_t)refresh_npanel(nmax) * RB * RB;   // diagonal 16x16 blocks of U11^-1
+    int* __restrict__ jint = reinterpret_cast<int*>(Usave + (size_t)refresh_npanel(nmax) * RB * RB);
+    int t = (int)threadIdx.x, lane = t % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(t / 64);
+    if (t == 0) jint[0] = 0;                             // set to 1 once the factors are complete
+
+    double* Dblk = reinterpret_cast<double*>(lds);       // [RB][LB] factored diagonal block
+    double* us = Dblk;                                   // [2][RB][16] panel J's U rows, by column tile (Dblk is done with)
+    double* Linv = Dblk + RB * LB;                       // [RB][LB] L11^-1
+    // the half panel by position (row of the panel's start) and column, on its
+    // way to and from registers; entry k of a row is at k ^ (row & 15)
+    double* R = Linv;                                    // [rup 16 of nmax][HB], at least Linv's size
+    double* pivabs = R + max(rup_i(nmax, 16) * HB, RB * LB);   // [nmax] |pivot|
+    double* redd = pivabs + nmax;                        // [3 * NWAVE]
+    unsigned short* phys = reinterpret_cast<unsigned short*>(redd + 3 * NWAVE);   // [rup 32 of nmax] logical -> physical row
+    unsigned short* snap = phys + rup_i(nmax, RB);       // the same as it was when the panel began
+    unsigned short* rowsite = snap + rup_i(nmax, RB);    // [nmax] label -> site (the solve kernel's LDS bounds ns far below 65536)
+    int* seen = reinterpret_cast<int*>(R);               // [nmax] times a label was met (at the start)
+    __shared__ int s_bad, s_occ, s_sing;
+
+    if (t == 0) { s_bad = 0; s_occ = 0; s_sing = 0; }
+    for (int k = t; k < N; k += TH) seen[k] = 0;
+    for (int r = t; r < rup_i(nmax, RB); r += TH) { phys[r] = (unsigned short)r; snap[r] = (unsigned short)r; }
+    __syncthreads();
+    for (int s = t; s < ns; s += TH) {
+        const int l = kap[s];
+        if (l < 0 || l > N) s_bad = 1;
+        else if (l > 0) {
+            rowsite[l - 1] = (unsigned short)s;
+            if (atomicAdd(&seen[l - 1], 1) != 0) s_bad = 1;
+            atomicAdd(&s_occ, 1);
+        }
+    }
+    __syncthreads();
+    if (s_bad || s_occ != N) {
+        if (t == 0) { a.status[w] = 2; atomicMin(a.failed, w); }
+        return;
+    }
+    {
+        // columns nc16..ldm-1 of M are read (as zeros) by the solve kernel
+        const int nz = ldm - nc16;
+        for (int idx = t; idx < nc16 * nz; idx += TH) M[(size_t)(idx / nz) * ldm + nc16 + idx % nz] = 0.0;
+        // and rows N..nc16-1 as zeros: here where no tile is stored whole
+        for (int idx = t; idx < (nc16 - N) * nc16; idx += TH) M[(size_t)(N + idx / nc16) * ldm + idx % nc16] = 0.0;
+    }
+
+    // Columns 32 Jn + 16 ct.. from U through the panels before np, rows from
+    // panel np on to M.  One wavefront; rows in the order of snap.
+    auto prepare = [&](int Jn, int np, int ct) __attribute__((always_inline)) {
+        if (RB * Jn + 16 * ct >= nc16) return;
+        asm volatile("" : "+v"(lane));
+        const int c = RB * Jn + 16 * ct + (lane & 15);
+        f64x4 acc[2 * NB];
+#pragma unroll
+        for (int i = 0; i < 2 * NB; ++i) {
+            acc[i] = f64x4{0, 0, 0, 0};
+            if (16 * i < nc16) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int pr = snap[16 * i + (lane >> 4) + 4 * g];
+                    acc[i][g] = (pr < N && c < N) ? UT[(size_t)rowsite[pr] * N + c] : 0.0;
+                }
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < NB - 1; ++p) {
+            if (p >= np) break;
+            asm volatile("" : "+v"(lane));
+            const int kr = lane >> 4, kc = lane & 15, cc = RB * Jn + 16 * ct + kc;
+            // the L operands of the first tiles below
+            double af[PD][RB / 4];
+#pragma unroll
+            for (int i = 0; i < PD; ++i) {
+                const int o = snap[min(16 * (2 * p + 2 + i), nc16 - 16) + kc] * ldm + kr + RB * p;
+#pragma unroll
+                for (int s = 0; s < RB / 4; ++s) af[(i + 2 * p + 2) % PD][s] = M[(size_t)o + 4 * s];
+            }
+            // U rows of panel p: L11^-1 (upper-right 16x16 block zero) times the block
+            const double* Li = Lsave + (size_t)p * RB * RB;
+            f64x4 u0 = {0, 0, 0, 0}, u1 = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                u0 = mfma16(Li[kc * RB + 4 * s + kr], acc[2 * p][s], u0);
+                u1 = mfma16(Li[(16 + kc) * RB + 4 * s + kr], acc[2 * p][s], u1);
+            }
+#pragma unroll
+            for (int s = 0; s < 4; ++s) u1 = mfma16(Li[(16 + kc) * RB + 16 + 4 * s + kr], acc[2 * p + 1][s], u1);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                M[(size_t)snap[RB * p + kr + 4 * g] * ldm + cc] = u0[g];
+                M[(size_t)snap[RB * p + 16 + kr + 4 * g] * ldm + cc] = u1[g];
+            }
+            // the accumulator layout is the B-operand layout; tiles past the
+            // rows go along (a branch here would have every load awaited)
+#pragma unroll
+            for (int i = 2 * p + 2; i < 2 * NB; ++i) {
+                const int o = snap[min(16 * (i + PD), nc16 - 16) + kc] * ldm + kr + RB * p;
+#pragma unroll
+                for (int s = 0; s < RB / 4; ++s) acc[i] = mfma16(-af[i % PD][s], s < 4 ? u0[s & 3] : u1[s & 3], acc[i]);
+                if (i + PD < 2 * NB) {   // tile i + PD's operands take their place
+#pragma unroll
+                    for (int s = 0; s < RB / 4; ++s) af[i % PD][s] = M[(size_t)o + 4 * s];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2 * NB; ++i) {
+            if (i >= 2 * np && 16 * i < nc16) {
+                asm volatile("" : "+v"(lane));
+                const int kr = lane >> 4, kc = lane & 15;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int pr = snap[16 * i + kr + 4 * g];
+                    const double v = pr < N ? acc[i][g] : 0.0;
+                    if (Jn == 0 && ct == 0) R[(16 * i + kr + 4 * g) * HB + (kc ^ (kr + 4 * g))] = v;
+                    else M[(size_t)pr * ldm + RB * Jn + 16 * ct + kc] = v;
+                }
+            }
+        }
+    };
+
+    // Wavefront 0: panel J (columns j0.., jb of them) factored in place; the
+    // row map; the diagonal block to Dblk.  False if a pivot is zero or not
+    // finite.
+    auto panel = [&](int j0, int jb) -> bool {
+        bool ok = true;
+        // lane + 64 q is a row's position; myp its physical row, myr the
+        // logical row it currently stands for
+        int myr[RPL], myp[RPL];
+#pragma unroll
+        for (int q = 0; q < RPL; ++q) {
+            myr[q] = j0 + lane + 64 * q;
+            myp[q] = myr[q] < N ? (int)snap[myr[q]] : -1;
+        }
+#pragma clang loop unroll(disable)
+        for (int h0 = j0; h0 < j0 + jb; h0 += HB) {
+            asm volatile("" : "+v"(lane));
+            const int hb = min(HB, N - h0);
+            const bool upper = h0 == j0;
+            {
+                double x[RPL][HB];
+#pragma unroll
+                for (int q = 0; q < RPL; ++q) {
+                    const int pos = min(lane + 64 * q, nc16 - 1 - j0);
+#pragma unroll
+                    for (int e = 0; e < HB; ++e) x[q][e] = R[pos * HB + (e ^ (pos & 15))];
+                }
+                asm volatile("" ::: "memory");
+#pragma clang loop unroll(full)
+                for (int jj = 0; jj < HB; ++jj) {
+                    if (jj < hb && ok) {
+                        const int kk = h0 + jj;
+                        // the largest key of pivot_key, its high and low words
+                        // in turn
+                        uint32_t hi[RPL], lo[RPL], bh = 0u, bl = 0u;
+#pragma unroll
+                        for (int q = 0; q < RPL; ++q) {
+                            const unsigned long long key =
+                                (myr[q] >= kk && myp[q] >= 0) ? pivot_key(x[q][jj], myr[q]) : 0ull;
+                            hi[q] = (uint32_t)(key >> 32);
+                            lo[q] = (uint32_t)key;
+                            bh = hi[q] > bh ? hi[q] : bh;
+                        }
+                        const uint32_t mhi = wave_max_u32(bh);
+#pragma unroll
+                        for (int q = 0; q < RPL; ++q) {
+                            lo[q] = hi[q] == mhi ? lo[q] : 0u;
+                            bl = lo[q] > bl ? lo[q] : bl;
+                        }
+                        const uint32_t mlo = wave_max_u32(bl);
+                        const int p = 4095 - (int)(mlo & 0xFFFu);
+                        // its row, entries of L and U, is final: it goes to
+                        // the diagonal block, where every lane reads it; the
+                        // registers it leaves are updated on with the others
+                        double* prow = Dblk + (kk - j0) * LB + (upper ? 0 : HB);
+#pragma unroll
+                        for (int q = 0; q < RPL; ++q) {
+                            if (lo[q] == mlo && hi[q] == mhi) {
+#pragma unroll
+                                for (int k = 0; k < HB; ++k) prow[k] = x[q][k];
+                            }
+                        }
+                        asm volatile("" ::: "memory");
+                        const double piv = prow[jj];
+                        double u[2][UC];
+#pragma unroll
+                        for (int e = 0; e < UC; ++e)
+                            if (jj + 1 + e < HB) u[0][e] = prow[jj + 1 + e];
+                        __builtin_amdgcn_sched_barrier(0);
+                        const uint32_t ph = (uint32_t)__builtin_amdgcn_readfirstlane((int)((unsigned long long)__double_as_longlong(piv) >> 32)) & 0x7FFFFFFFu;
+                        const uint32_t pl = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)__double_as_longlong(piv));
+                        if ((ph | pl) == 0u || ph >= 0x7FF00000u) {
+                            ok = false;
+                        } else {
+                            if (lane == 0) pivabs[kk] = fabs(piv);
+                            const double rp = rcp_f64(piv);
+#pragma unroll
+                            for (int q = 0; q < RPL; ++q) {
+                                const int r = myr[q];
+                                myr[q] = (r == p) ? kk : (r == kk ? p : r);
+                                x[q][jj] *= rp;
+                            }
+#pragma unroll
+                            for (int c = 0; c < (HB + UC - 1) / UC; ++c) {
+                                // UC columns at a time, the next ones' pivot
+                                // row entries under way
+#pragma unroll
+                                for (int e = 0; e < UC; ++e)
+                                    if (jj + 1 + (c + 1) * UC + e < HB) u[(c + 1) & 1][e] = prow[jj + 1 + (c + 1) * UC + e];
+                                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                                for (int e = 0; e < UC; ++e) {
+                                    const int k = jj + 1 + c * UC + e;
+                                    if (k < HB) {
+#pragma unroll
+                                        for (int q = 0; q < RPL; ++q) x[q][k] -= x[q][jj] * u[c & 1][e];
+                                    }
+                                }
+                            }
+                        }
+                        asm volatile("" ::: "memory");
+                    }
+                }
+                // the row map; the rows by position, and from there back to
+                // the physical rows; the pivot rows from the diagonal block
+                int to[RPL];
+#pragma unroll
+                for (int q = 0; q < RPL; ++q) {
+                    if (myp[q] >= 0) phys[myr[q]] = (unsigned short)myp[q];
+                    to[q] = (myp[q] >= 0 && myr[q] >= h0 + hb) ? myp[q] : -1;
+                    const int pos = lane + 64 * q;
+                    if (pos < nc16 - j0) {
+#pragma unroll
+                        for (int e = 0; e < HB; ++e) R[pos * HB + (e ^ (pos & 15))] = x[q][e];
+                    }
+                }
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int q = 0; q < RPL; ++q) {
+                    if (q == 0 || j0 + 64 * q < N) {
+                        double2 v[8];
+                        int pr[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const int r = 8 * i + (lane >> 3), pos = min(64 * q + r, nc16 - 1 - j0), e = 2 * (lane & 7);
+                            v[i] = make_double2(R[pos * HB + (e ^ (pos & 15))], R[pos * HB + ((e + 1) ^ (pos & 15))]);
+                            pr[i] = __shfl(to[q], r, 64);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i)
+                            if (pr[i] >= 0) *reinterpret_cast<double2*>(M + (size_t)pr[i] * ldm + h0 + 2 * (lane & 7)) = v[i];
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < HB; i += 8) {
+                    const int r = i + (lane >> 3);
+                    const double* d = Dblk + (h0 - j0 + r) * LB + (upper ? 0 : HB) + 2 * (lane & 7);
+                    if (r < hb) *reinterpret_cast<double2*>(M + (size_t)phys[h0 + r] * ldm + h0 + 2 * (lane & 7)) = make_double2(d[0], d[1]);
+                }
+            }
+            if (!ok) return false;
+            const int kr = lane >> 4, kc = lane & 15;
+            if (upper && jb > HB) {
+                // the first half's 16 pivot rows in the second half's columns,
+                // u_k = a_k - sum_{j<k} l_kj u_j in the order of j: register g
+                // holds rows 4g..4g+3, which take the rows of the group among
+                // themselves and then pass on to the groups below as one MFMA
+                // slice
+                const int r0 = j0 + HB, cc = r0 + kc;
+                f64x4 u;
+                {
+                    int mo[4];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        mo[g] = phys[j0 + 4 * g + kr] * ldm + cc;
+                        u[g] = M[mo[g]];
+                    }
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                        for (int j = 0; j < 3; ++j) {
+                            const double uj = __shfl(u[s], 16 * j + kc, 64);
+                            const double l = Dblk[(4 * s + kr) * LB + 4 * s + j];
+                            if (kr > j) u[s] -= l * uj;
+                        }
+                        if (s < 3) {
+                            const f64x4 v = mfma16(-Dblk[kc * LB + 4 * s + kr], u[s], u);
+#pragma unroll
+                            for (int g = 0; g < 4; ++g)
+                                if (g > s) u[g] = v[g];
+                        }
+                    }
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        M[mo[g]] = u[g];
+                        Dblk[(4 * g + kr) * LB + HB + kc] = u[g];
+                    }
+                }
+                // all positions: a -= l u, TM row tiles at once (a tile past
+                // the last repeats it and is not stored; a row that has been a
+                // pivot gets nothing of use)
+                constexpr int TM = NB > 4 ? 4 : 2;
+                const int ntr = (nc16 - j0) / 16;
+#pragma clang loop unroll(disable)
+                for (int tb = 0; tb < ntr; tb += TM) {
+                    double af[TM][4];
+                    f64x4 v[TM];
+#pragma unroll
+                    for (int e = 0; e < TM; ++e) {
+                        const int ti = min(tb + e, ntr - 1);
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) v[e][g] = M[(size_t)snap[j0 + 16 * ti + kr + 4 * g] * ldm + cc];
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) af[e][s] = R[(16 * ti + kc) * HB + ((4 * s + kr) ^ kc)];
+                    }
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+                        for (int e = 0; e < TM; ++e) v[e] = mfma16(-af[e][s], u[s], v[e]);
+                    }
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int e = 0; e < TM; ++e) {
+                        if (tb + e < ntr) {
+#pragma unroll
+                            for (int g = 0; g < 4; ++g) R[(16 * (tb + e) + kr + 4 * g) * HB + (kc ^ (kr + 4 * g))] = v[e][g];
+                        }
+                    }
+                }
+                asm volatile("" ::: "memory");
+            }
+        }
+        // what the halves have not put into the diagonal block: columns 0..15
+        // of rows 16.. (rows moved in the second half), and rows jb.. as unit
+        // rows
+        double lc[RB * HB / 128];
+#pragma unroll
+        for (int e = 0; e < RB * HB / 128; ++e)
+            lc[e] = M[(size_t)phys[min(j0 + HB + 4 * e + (lane >> 4), N - 1)] * ldm + j0 + (lane & 15)];
+#pragma unroll
+        for (int e = 0; e < RB * HB / 64; ++e) {
+            const int i = 4 * e + (lane >> 4), k = lane & 15;
+            if (i >= HB) Dblk[i * LB + k] = i < jb ? lc[e >= 4 ? e - 4 : 0] : 0.0;
+            else if (i >= jb) Dblk[i * LB + k] = k == i ? 1.0 : 0.0;
+            if (i >= jb || jb <= HB) Dblk[i * LB + HB + k] = i >= HB && k == i - HB ? 1.0 : 0.0;
+        }
+        return true;
+    };
+
+    bool singular = false;
+    if (LUW == 2 || wave > 0) prepare(0, 0, LUW == 2 ? wave : wave - 1);
+    __syncthreads();
+#pragma clang loop unroll(disable)
+    for (int j0 = 0; j0 < N; j0 += RB) {
+        const int J = j0 / RB, jb = min(RB, N - j0);
+        if (wave == 0) {
+            const bool ok = panel(j0, jb);
+            if (!ok && lane == 0) s_sing = 1;
+        } else if (j0 + RB < N) {
+            if constexpr (LUW == 2) {
+#pragma clang loop unroll(disable)
+                for (int ct = 0; ct < 2; ++ct) prepare(J + 1, J, ct);
+            } else {
+                prepare(J + 1, J, wave - 1);
+            }
+        }
+        __syncthreads();
+        if (s_sing) { singular = true; break; }
+        // opaque once a panel: the many addresses made of the lane are formed
+        // where they are used, not kept (and spilled) across the panels
+        asm volatile("" : "+v"(t), "+v"(lane));
+        const int kr = lane >> 4, kc = lane & 15;
+        // the 16x16 diagonal blocks of U11^-1 (all the solve kernel reads) and
+        // of L11^-1; then the lower-left block of L11^-1, -Lb^-1 Lc La^-1, on
+        // MFMA (Lc: rows 16.., columns ..15 of L11); the upper-right block is
+        // zero
+        if (wave == 0) {
+            unit_lower_inverse16x2(Dblk, Linv, jb, lane);
+            f64x4 tq = {0, 0, 0, 0}, xq = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) tq = mfma16(Dblk[(16 + kc) * LB + 4 * s + kr], Linv[(4 * s + kr) * LB + kc], tq);
+            // the product's accumulator layout is the B-operand layout
+#pragma unroll
+            for (int s = 0; s < 4; ++s) xq = mfma16(Linv[(16 + kc) * LB + 16 + 4 * s + kr], tq[s], xq);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) Linv[(16 + kr + 4 * g) * LB + kc] = -xq[g];
+        } else if (wave == 1) {
+            upper_inverse16x2(Dblk, Usave + (size_t)J * RB * RB, RB, lane);
+        }
+        if (wave == LUW - 1) {
+            for (int idx = lane; idx < 256; idx += 64) Linv[(idx / 16) * LB + 16 + idx % 16] = 0.0;
+            for (int r = j0 + lane; r < nc16; r += 64) snap[r] = phys[r];
+        }
+        __syncthreads();
+        for (int idx = t; idx < RB * RB; idx += TH) Lsave[(size_t)J * RB * RB + idx] = Linv[(idx / RB) * LB + idx % RB];
+        const int c0 = j0 + RB;
+        if (c0 >= N) break;
+        // panel J's step on the next panel's columns: TQ row tiles of a
+        // wavefront at once, the first ones' operands under way before the U
+        // rows they wait for (a tile past the last repeats it and is not
+        // stored; two below 129 columns would spill)
+        const bool two = c0 + 16 < nc16;
+        const int ntr = (nc16 - c0) / 16;
+        constexpr int TQ = NB > 4 ? 2 : 1;
+        double af[TQ][RB / 4];
+        f64x4 v0[TQ], v1[TQ];
+        int mo[TQ][4];
+        auto operands = [&](int tb) {
+#pragma unroll
+            for (int e = 0; e < TQ; ++e) {
+                const int ti = min(tb + e * LUW, ntr - 1);
+                const int pa = snap[c0 + 16 * ti + kc] * ldm + j0 + kr;
+#pragma unroll
+                for (int s = 0; s < RB / 4; ++s) af[e][s] = M[pa + 4 * s];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    mo[e][g] = snap[c0 + 16 * ti + kr + 4 * g] * ldm + c0 + kc;
+                    v0[e][g] = M[mo[e][g]];
+                    v1[e][g] = two ? M[mo[e][g] + 16] : 0.0;
+                }
+            }
+        };
+        // the U rows ...
+        if (wave == 0 || (wave == 1 && two)) {
+            const int c = c0 + 16 * wave + kc;
+            double b[RB / 4];
+            int bo[RB / 4];
+#pragma unroll
+            for (int s = 0; s < RB / 4; ++s) {
+                bo[s] = phys[j0 + 4 * s + kr] * ldm + c;
+                b[s] = M[bo[s]];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            operands(wave);
+            __builtin_amdgcn_sched_barrier(0);
+            f64x4 u0 = {0, 0, 0, 0}, u1 = {0, 0, 0, 0};
+#pragma unroll
+            for (int s = 0; s < RB / 4; ++s) {
+                if (s < 4) u0 = mfma16(Linv[kc * LB + 4 * s + kr], b[s], u0);
+                u1 = mfma16(Linv[(16 + kc) * LB + 4 * s + kr], b[s], u1);
+            }
+            double* ub = us + wave * RB * 16;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                ub[(kr + 4 * g) * 16 + kc] = u0[g];
+                ub[(16 + kr + 4 * g) * 16 + kc] = u1[g];
+                M[bo[g]] = u0[g];
+                M[bo[4 + g]] = u1[g];
+            }
+        } else {
+            operands(wave);
+        }
+        __syncthreads();
+        // ... and the rows below
+        {
+            double b0[RB / 4], b1[RB / 4];
+#pragma unroll
+            for (int s = 0; s < RB / 4; ++s) {
+                b0[s] = us[(4 * s + kr) * 16 + kc];
+                b1[s] = two ? us[RB * 16 + (4 * s + kr) * 16 + kc] : 0.0;
+            }
+#pragma clang loop unroll(disable)
+            for (int tb = wave; tb < ntr; tb += TQ * LUW) {
+                if (tb != wave) operands(tb);
+#pragma unroll
+                for (int s = 0; s < RB / 4; ++s) {
+#pragma unroll
+                    for (int e = 0; e < TQ; ++e) {
+                        v0[e] = mfma16(-af[e][s], b0[s], v0[e]);
+                        v1[e] = mfma16(-af[e][s], b1[s], v1[e]);
+                    }
+                }
+#pragma unroll
+                for (int e = 0; e < TQ; ++e) {
+                    const int ti = tb + e * LUW;
+                    if (ti < ntr) {
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            R[(16 * ti + kr + 4 * g) * HB + (kc ^ (kr + 4 * g))] = v0[e][g];
+                            if (two) M[mo[e][g] + 16] = c0 + 16 * ti + kr + 4 * g < N ? v1[e][g] : 0.0;
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    double logdet = 0.0, pmin = INFINITY, pmax = 0.0;
+    if (!singular) {
+        // 64 pivots a wavefront, the partial sums added in order
+#pragma clang loop unroll(disable)
+        for (int g = wave; g < NWAVE; g += LUW) {
+            const int k = 64 * g + lane;
+            const double v = k < N ? pivabs[k] : 0.0;
+            double ls = k < N ? log(v) : 0.0, mn = k < N ? v : INFINITY, mx = v;
+            for (int o = 32; o > 0; o >>= 1) {
+                ls += __shfl_xor(ls, o, 64);
+                mn = fmin(mn, __shfl_xor(mn, o, 64));
+                mx = fmax(mx, __shfl_xor(mx, o, 64));
+            }
+            if (lane == 0) { redd[g] = ls; redd[NWAVE + g] = mn; redd[2 * NWAVE + g] = mx; }
+        }
+        __syncthreads();
+        for (int q = 0; q < NWAVE; ++q) {
+            logdet += redd[q];
+            pmin = fmin(pmin, redd[NWAVE + q]);
+            pmax = fmax(pmax, redd[2 * NWAVE + q]);
+        }
+    }
+    if (!singular && pmin < a.pivot_tol * pmax) singular = true;
+    if (singular) {
+        if (t == 0) { a.status[w] = 1; atomicMin(a.failed, w); }
+        return;
+    }
+    // logical row k < N holds label phys[k]; W is formed by the solve kernel
+    for (int k = t; k < N; k += TH) jint[1 + k] = phys[k];
+    if (t == 0) {
+        a.logdet[(size_t)w * 2 + spin] = logdet;
+        if (a.write_w) a.stiff[(size_t)w * 2 + spin] = pmin < kStiffTol * pmax;
+        if (a.write_w && spin == 0) { a.npend[w] = 0; a.acc_since[w] = 0; }
+        jint[0] = 1;
+    }
+}
+
+template <typename T, int RPT>
+__global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_refresh_blocked(RefreshArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int job = (int)blockIdx.x;
     if (job >= a.njobs) return;
@@ -255,8 +868,8 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
     // of site s), those of the first ns_out sites only, the rows W is made
     // of.  The pivots come from the rows of tildeU, so the others are not
     // needed.
-    const int nkeep = (FULL && a.cplx_out) ? a.ns_out : ns;
-    const int nE = (FULL && a.cplx_out) ? a.ns_out - (spin ? a.ndn_out : a.nup_out) : ns - N;
+    const int nkeep = a.cplx_out ? a.ns_out : ns;
+    const int nE = a.cplx_out ? a.ns_out - (spin ? a.ndn_out : a.nup_out) : ns - N;
     const int nr16 = rup_i(N + nE, 16);  // logical rows that carry data
     const int nc16 = rup_i(N, 16);       // columns that carry data
     const int m16 = rup_i(nE, 16);       // empty-site rows, padded
@@ -264,12 +877,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
     const int* __restrict__ kap = (spin ? a.kdn : a.kup) + (size_t)w * ns;
     double* __restrict__ M = a.ws + (size_t)job * refresh_ws_job(ns, nmax);
     double* __restrict__ Lsave = M + (size_t)nrows * ldm;   // [npanel][RB][RB] inverses of L11
-    double* __restrict__ Usave = Lsave + (size_t)refresh_npanel(nmax) * RB * RB;   // inverses of U11
-    int* __restrict__ jint = reinterpret_cast<int*>(Usave + (size_t)refresh_npanel(nmax) * RB * RB);
     const int t = (int)threadIdx.x, wave = t / 64, lane = t % 64;
-    if (!FULL && t == 0) jint[0] = 0;                       // set to 1 once the factors are complete
-    // logical rows carrying data: all of M, or only tildeU
-    const int nrl = FULL ? nr16 : rup_i(N, 16);
 
     // ---- LDS carve-up ----------------------------------------------------
     double* cand = reinterpret_cast<double*>(lds);          // [2][NWAVE][RB]
@@ -278,7 +886,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
     double* Dblk = reinterpret_cast<double*>(candk + 2 * NWAVE);    // [RB][LB] factored diagonal block
     double* Linv = Dblk + RB * LB;                          // [RB][LB] U11^-1, then L11^-1
     double* stage = Linv + RB * LB;                         // W scatter block (single kernel)
-    const int stage_len = FULL ? kStoreBlock * (nc16 | 1) : 0;
+    const int stage_len = kStoreBlock * (nc16 | 1);
     double* pivabs = stage + stage_len;                     // [nmax] |pivot|
     double* redd = pivabs + nmax;                           // [3 * NWAVE]
     int* wsum = reinterpret_cast<int*>(redd + 3 * NWAVE);   // [NWAVE]
@@ -330,16 +938,11 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
         if (t == 0) { a.status[w] = 2; atomicMin(a.failed, w); }
         return;
     }
-    if (!FULL) {
-        // columns nc16..ldm-1 of M are read (as zeros) by the solve kernel
-        const int nz = ldm - nc16;
-        for (int idx = t; idx < nrl * nz; idx += RT) M[(size_t)(idx / nz) * ldm + nc16 + idx % nz] = 0.0;
-    }
     // M is never filled from U up front: the first panel (j0 = 0) reads its
     // operands straight from U (L2-resident, shared by every job) and every
     // later read of M finds values written by an earlier step.
     auto u_at = [&](int prow, int col) -> double {
-        return (prow < (FULL ? N + nE : N) && col < N) ? UT[(size_t)rowsite[prow] * N + col] : 0.0;
+        return (prow < N + nE && col < N) ? UT[(size_t)rowsite[prow] * N + col] : 0.0;
     };
 
     // ---- 1. blocked LU ---------------------------------------------------
@@ -447,70 +1050,32 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
         for (int i = jb + t; i < RB; i += RT) {
             for (int c = 0; c < RB; ++c) Dblk[i * LB + c] = (c == i) ? 1.0 : 0.0;
         }
-        if (!FULL) {
-            // padding rows N..nrl-1 (phys[r] = r) enter the trailing update
-            // as zero rows; nothing reads their results
-            for (int r = N + t; r < nrl; r += RT) {
-                for (int c = 0; c < RB; ++c) M[(size_t)r * ldm + j0 + c] = 0.0;
+        __syncthreads();
+        // U11^-1, applied to the empty-site rows, whose panel slice solves
+        // x U11 = a  ->  x = a U11^-1
+        upper_inverse(Dblk, Linv, LB, 0);
+        __syncthreads();
+        const int ntr = m16 / 16;
+        for (int ti = wave; ti < ntr; ti += NWAVE) {
+            const int ra = N + 16 * ti + (lane & 15);
+            f64x4 y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
+#pragma unroll
+            for (int s2 = 0; s2 < RB / 4; ++s2) {
+                const int k = 4 * s2 + (lane >> 4);
+                const double av = j0 == 0 ? u_at(ra, k) : M[(size_t)ra * ldm + j0 + k];
+                y0 = mfma16(av, Linv[k * LB + (lane & 15)], y0);
+                y1 = mfma16(av, Linv[k * LB + 16 + (lane & 15)], y1);
+            }
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const size_t row = (size_t)(N + 16 * ti + (lane >> 4) + 4 * g) * ldm + j0;
+                M[row + (lane & 15)] = y0[g];
+                M[row + 16 + (lane & 15)] = y1[g];
             }
         }
         __syncthreads();
-        // U11^-1: kept for the solve kernel (computed by wavefront 0 while
-        // wavefront 1 forms L11^-1), or applied here to the empty-site rows,
-        // whose panel slice solves x U11 = a  ->  x = a U11^-1
-        if constexpr (!FULL) {
-            // the 16x16 diagonal blocks of U11^-1 (all the solve kernel reads)
-            // and of L11^-1, one per wavefront; then the lower-left block of
-            // L11^-1, -Lb^-1 Lc La^-1, on MFMA (Lc: rows 16.., columns ..15 of
-            // L11); the upper-right block is zero
-            double* Us = Usave + (size_t)(j0 / RB) * RB * RB;
-            upper_inverse16(Dblk, Us, RB, 0, 0);
-            upper_inverse16(Dblk, Us, RB, 16, 1);
-            unit_lower_inverse16(Dblk, Linv, 0, jb, 2);
-            unit_lower_inverse16(Dblk, Linv, 16, jb, 3);
-            __syncthreads();
-            if (wave == 0) {
-                f64x4 tq = {0, 0, 0, 0}, xq = {0, 0, 0, 0};
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    const int k = 4 * s + (lane >> 4);
-                    tq = mfma16(Dblk[(16 + (lane & 15)) * LB + k], Linv[k * LB + (lane & 15)], tq);
-                }
-                // the product's accumulator layout is the B-operand layout
-#pragma unroll
-                for (int s = 0; s < 4; ++s)
-                    xq = mfma16(Linv[(16 + (lane & 15)) * LB + 16 + 4 * s + (lane >> 4)], tq[s], xq);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) Linv[(16 + (lane >> 4) + 4 * g) * LB + (lane & 15)] = -xq[g];
-            } else if (wave == 1) {
-                for (int idx = lane; idx < 256; idx += 64) Linv[(idx / 16) * LB + 16 + idx % 16] = 0.0;
-            }
-            __syncthreads();
-        } else {
-            upper_inverse(Dblk, Linv, LB, 0);
-            __syncthreads();
-            const int ntr = m16 / 16;
-            for (int ti = wave; ti < ntr; ti += NWAVE) {
-                const int ra = N + 16 * ti + (lane & 15);
-                f64x4 y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
-#pragma unroll
-                for (int s2 = 0; s2 < RB / 4; ++s2) {
-                    const int k = 4 * s2 + (lane >> 4);
-                    const double av = j0 == 0 ? u_at(ra, k) : M[(size_t)ra * ldm + j0 + k];
-                    y0 = mfma16(av, Linv[k * LB + (lane & 15)], y0);
-                    y1 = mfma16(av, Linv[k * LB + 16 + (lane & 15)], y1);
-                }
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const size_t row = (size_t)(N + 16 * ti + (lane >> 4) + 4 * g) * ldm + j0;
-                    M[row + (lane & 15)] = y0[g];
-                    M[row + 16 + (lane & 15)] = y1[g];
-                }
-            }
-            __syncthreads();
-            unit_lower_inverse(Dblk, Linv, jb, 0);
-            __syncthreads();
-        }
+        unit_lower_inverse(Dblk, Linv, jb, 0);
+        __syncthreads();
         for (int idx = t; idx < RB * RB; idx += RT)
             Lsave[(size_t)(j0 / RB) * RB * RB + idx] = Linv[(idx / RB) * LB + idx % RB];
         const int c0 = j0 + RB;
@@ -522,7 +1087,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
         // panel, -1 for padding rows, in M afterwards); elsewhere that
         // spills, and the operands are loaded per block.
         const int ntc = (nc16 - c0) / 16;
-        if constexpr (FULL && RPT <= 2) {
+        if constexpr (RPT <= 2) {
             int bofs[RB / 4];
 #pragma unroll
             for (int s = 0; s < RB / 4; ++s) {
@@ -591,22 +1156,22 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
         // register peak) and spills elsewhere.  The C operands come from U in
         // the first panel and from M afterwards, a loop for each, so that
         // only one set of row offsets is live.
-        constexpr int TG = (FULL && RPT == 2) ? 2 : 1;
+        constexpr int TG = RPT == 2 ? 2 : 1;
         const int r0 = c0;
-        const int ntr = (nrl - r0) / 16;
+        const int ntu = (nr16 - r0) / 16;
         int uofs[RB / 4];   // U12 operand rows: offsets in M
 #pragma unroll
         for (int s = 0; s < RB / 4; ++s) uofs[s] = phys[j0 + 4 * s + (lane >> 4)] * ldm + c0 + (lane & 15);
         auto tiles = [&](auto first_panel) {
             constexpr bool FIRST = decltype(first_panel)::value;
-            for (int tb = wave; tb < ntr; tb += TG * NWAVE) {
+            for (int tb = wave; tb < ntu; tb += TG * NWAVE) {
                 double af[TG][RB / 4];
                 int mofs[TG][4];   // C rows: offsets in M
                 int cofs[TG][4];   // first panel: the rows' offsets in U, -1 for padding rows
 #pragma unroll
                 for (int k = 0; k < TG; ++k) {
-                    // a tile past ntr repeats the last one and is never stored
-                    const int ti = min(tb + k * NWAVE, ntr - 1);
+                    // a tile past ntu repeats the last one and is never stored
+                    const int ti = min(tb + k * NWAVE, ntu - 1);
                     const int pa = phys[r0 + 16 * ti + (lane & 15)];
 #pragma unroll
                     for (int s = 0; s < RB / 4; ++s) af[k][s] = -M[(size_t)pa * ldm + j0 + 4 * s + (lane >> 4)];
@@ -614,7 +1179,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
                     for (int g = 0; g < 4; ++g) {
                         const int pr = phys[r0 + 16 * ti + (lane >> 4) + 4 * g];
                         mofs[k][g] = pr * ldm + c0 + (lane & 15);
-                        if constexpr (FIRST) cofs[k][g] = pr < (FULL ? N + nE : N) ? rowsite[pr] * N : -1;
+                        if constexpr (FIRST) cofs[k][g] = pr < N + nE ? rowsite[pr] * N : -1;
                     }
                 }
                 auto cval = [&](int k, int g, int tj) -> double {
@@ -651,7 +1216,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
                     }
 #pragma unroll
                     for (int k = 0; k < TG; ++k) {
-                        if (tb + k * NWAVE < ntr) {
+                        if (tb + k * NWAVE < ntu) {
 #pragma unroll
                             for (int g = 0; g < 4; ++g) M[(size_t)mofs[k][g] + 16 * tj] = acc[k][g];
                         }
@@ -698,12 +1263,6 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(FULL ? 
         a.logdet[(size_t)w * 2 + spin] = logdet;
         if (a.write_w) a.stiff[(size_t)w * 2 + spin] = pmin < kStiffTol * pmax;
         if (a.write_w && spin == 0) { a.npend[w] = 0; a.acc_since[w] = 0; }
-    }
-    if constexpr (!FULL) {
-        // logical row c < N holds label phys[c]; W is formed by k_refresh_solve
-        for (int c = t; c < N; c += RT) jint[1 + c] = phys[c];
-        if (t == 0) jint[0] = 1;
-        return;
     }
     // logical row c < N holds label phys[c]
     for (int c = t; c < N; c += RT) pinv[phys[c]] = c;
@@ -937,8 +1496,7 @@ __device__ __forceinline__ void solve_stage(const double* M, int ldm, const int*
     }
 }
 
-// The empty-site rows of W from the factors of k_refresh_blocked<FULL =
-// false>: W[s][:] = U[s][:] tildeU^-1 = ((U[s][:] U1^-1) L1^-1) P.
+// The empty-site rows of W from the factors of k_lu: W[s][:] = U[s][:] tildeU^-1 = ((U[s][:] U1^-1) L1^-1) P.
 //
 // Each wavefront takes 16 empty sites and keeps the transposed rows as
 // 16x16 tiles T_J (labels 16J.. of the 16 sites) in MFMA accumulator layout:
@@ -1201,9 +1759,9 @@ static size_t solve_lds_bytes(int ns, int nt) { return (size_t)(nt * 16 + NWAVE 
 
 size_t refresh_ws_doubles_per_job(int ns, int nmax) { return refresh_ws_job(ns, nmax); }
 
-static size_t refresh_lds_bytes(int ns, int nup, int ndn, bool full = true) {
+static size_t refresh_lds_bytes(int ns, int nup, int ndn) {
     const int nmax = nup > ndn ? nup : ndn;
-    const int stage = !full ? 0 : kStoreBlock * (rup_i(nmax, 16) | 1);
+    const int stage = kStoreBlock * (rup_i(nmax, 16) | 1);
     const size_t dbl = (size_t)(2 * NWAVE * RB + 2 * NWAVE + 2 * RB * LB + stage + nmax + 3 * NWAVE) * sizeof(double);
     const size_t ints = (size_t)(NWAVE + refresh_nrows(ns) + 2 * ns + nmax) * sizeof(int);
     return dbl + ints + 16;
@@ -1218,11 +1776,22 @@ static hipError_t set_lds_limit(const void* fn, size_t lds) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
-template <typename T, int RPT, bool FULL>
-static hipError_t launch_lu(const RefreshArgs& a, size_t lds, hipStream_t s) {
-    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, RPT, FULL>), lds);
+template <typename T, int RPT>
+static hipError_t launch_single(const RefreshArgs& a, size_t lds, hipStream_t s) {
+    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, RPT>), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_refresh_blocked<T, RPT, FULL>), dim3(a.njobs), dim3(RT), lds, s, a);
+    hipLaunchKernelGGL((k_refresh_blocked<T, RPT>), dim3(a.njobs), dim3(RT), lds, s, a);
+    return hipGetLastError();
+}
+
+static size_t lu_lds_bytes(int nmax) {
+    const int r = rup_i(nmax, 16) * (RB / 2) > RB * LB ? rup_i(nmax, 16) * (RB / 2) : RB * LB;
+    return (size_t)(RB * LB + r + nmax + 3 * NWAVE) * sizeof(double) + (size_t)(2 * rup_i(nmax, RB) + nmax) * 2;
+}
+
+template <int NB, int LUW>
+static hipError_t launch_lu(const RefreshArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL((k_lu<NB, LUW>), dim3(a.njobs), dim3(64 * LUW), lu_lds_bytes(a.nmax), s, a);
     return hipGetLastError();
 }
 
@@ -1254,7 +1823,16 @@ template <typename T>
 static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t s) {
     const int tiles = solve_tiles(a.ns, a.nmax);
     if (tiles) {
-        hipError_t e = launch_lu<T, 1, false>(a, refresh_lds_bytes(a.ns, a.nup, a.ndn, false), s);
+        hipError_t e;
+        switch (refresh_npanel(a.nmax)) {   // one instance per number of panels: tiles past the rows cost their products
+            case 0: case 1: case 2: e = launch_lu<2, 2>(a, s); break;
+            case 3: e = launch_lu<3, 2>(a, s); break;
+            case 4: e = launch_lu<4, 2>(a, s); break;
+            case 5: e = launch_lu<5, 3>(a, s); break;
+            case 6: e = launch_lu<6, 3>(a, s); break;
+            case 7: e = launch_lu<7, 3>(a, s); break;
+            default: e = launch_lu<8, 2>(a, s); break;
+        }
         if (e != hipSuccess) return e;
         switch (tiles) {
             case 2: return launch_solve<T, 2>(a, s);
@@ -1268,9 +1846,9 @@ static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t
         }
     }
     switch (refresh_rows_per_thread(a.nmax)) {
-        case 1: return launch_lu<T, 1, true>(a, lds, s);
-        case 2: return launch_lu<T, 2, true>(a, lds, s);
-        case 3: return launch_lu<T, 3, true>(a, lds, s);
+        case 1: return launch_single<T, 1>(a, lds, s);
+        case 2: return launch_single<T, 2>(a, lds, s);
+        case 3: return launch_single<T, 3>(a, lds, s);
         default: return hipErrorInvalidValue;   // rejected by refresh_supported
     }
 }
