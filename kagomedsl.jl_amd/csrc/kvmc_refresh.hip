@@ -17,13 +17,18 @@
 //   (block rows of the factors staged through LDS, shared by the four
 //   wavefronts).  W[s][phys[c]] = x[c]; occupied rows of W are unit rows.
 //
-// N > 256 (register tiles would not fit): one kernel of a 256-thread
-// workgroup per (walker, spin), k_refresh_blocked, right-looking: the panel in
-// registers (one row per thread and more), one barrier per pivot column to
-// publish each wavefront's best candidate row, U12 = L11^-1 A12 and the
-// trailing update on FP64 MFMA (v_mfma_f64_16x16x4f64).  It factors the tall
-// matrix [tildeU ; U_empty] (rows >= N end as L2 = U_empty U1^-1), solves
-// X L1 = L2 panel by panel and writes W_empty = X P through LDS.
+// 256 < N <= 512 (mostly the real form of complex orbitals): two kernels again,
+//   k_refresh_blocked<FULL = false>, a 256-thread workgroup per (walker, spin),
+//   right-looking: the panel in registers (two rows per thread), one barrier
+//   per pivot column to publish each wavefront's best candidate row, U12 =
+//   L11^-1 A12 and the trailing update on FP64 MFMA
+//   (v_mfma_f64_16x16x4f64); then k_refresh_solve2, the solve with its tiles
+//   split over two wavefronts.
+//
+// N > 512 (or more sites than the solves' LDS takes): one kernel,
+// k_refresh_blocked<FULL = true>, which factors the tall matrix [tildeU ;
+// U_empty] (rows >= N end as L2 = U_empty U1^-1), solves X L1 = L2 panel by
+// panel and writes W_empty = X P through LDS.
 #include "kvmc_internal.hpp"
 
 #include <math.h>
@@ -56,8 +61,9 @@ __host__ __device__ inline int solve_nt(int nmax) {
     const int nt = (nmax + 15) / 16;
     return nt <= 16 ? (nt + 1) / 2 * 2 : 0;
 }
-// Row stride of M: whole 16 * NT rows for the solve kernel's row loads.
-__host__ __device__ inline int refresh_ldm(int nmax) { return solve_nt(nmax) ? 16 * solve_nt(nmax) : rup_i(nmax, 32); }
+// Row stride of M: whole 16 * NT rows for the solve kernel's row loads (up to
+// 512: whole pairs of 32-label blocks).
+__host__ __device__ inline int refresh_ldm(int nmax) { return solve_nt(nmax) ? 16 * solve_nt(nmax) : rup_i(nmax, nmax <= 512 ? 64 : 32); }
 __host__ __device__ inline int refresh_npanel(int nmax) { return (nmax + RB - 1) / RB; }
 // Work doubles per job: the padded tall matrix, the saved 32x32 inverses of
 // the diagonal blocks of L1 and of U1, then ints: [0] factorisation ok flag,
@@ -853,7 +859,7 @@ __global__ void __launch_bounds__(64 * LUW) __attribute__((amdgpu_waves_per_eu(N
     }
 }
 
-template <typename T, int RPT>
+template <typename T, int RPT, bool FULL>
 __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_refresh_blocked(RefreshArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int job = (int)blockIdx.x;
@@ -869,7 +875,8 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
     // of.  The pivots come from the rows of tildeU, so the others are not
     // needed.
     const int nkeep = a.cplx_out ? a.ns_out : ns;
-    const int nE = a.cplx_out ? a.ns_out - (spin ? a.ndn_out : a.nup_out) : ns - N;
+    const int nEmpty = a.cplx_out ? a.ns_out - (spin ? a.ndn_out : a.nup_out) : ns - N;
+    const int nE = FULL ? nEmpty : 0;    // rows below tildeU that are carried along
     const int nr16 = rup_i(N + nE, 16);  // logical rows that carry data
     const int nc16 = rup_i(N, 16);       // columns that carry data
     const int m16 = rup_i(nE, 16);       // empty-site rows, padded
@@ -877,6 +884,9 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
     const int* __restrict__ kap = (spin ? a.kdn : a.kup) + (size_t)w * ns;
     double* __restrict__ M = a.ws + (size_t)job * refresh_ws_job(ns, nmax);
     double* __restrict__ Lsave = M + (size_t)nrows * ldm;   // [npanel][RB][RB] inverses of L11
+    double* __restrict__ Usave = Lsave + (size_t)refresh_npanel(nmax) * RB * RB;   // inverses of U11 (FULL false)
+    int* __restrict__ jint = reinterpret_cast<int*>(Usave + (size_t)refresh_npanel(nmax) * RB * RB);
+    if (!FULL && threadIdx.x == 0) jint[0] = 0;             // set to 1 once the factors are complete
     const int t = (int)threadIdx.x, wave = t / 64, lane = t % 64;
 
     // ---- LDS carve-up ----------------------------------------------------
@@ -886,7 +896,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
     double* Dblk = reinterpret_cast<double*>(candk + 2 * NWAVE);    // [RB][LB] factored diagonal block
     double* Linv = Dblk + RB * LB;                          // [RB][LB] U11^-1, then L11^-1
     double* stage = Linv + RB * LB;                         // W scatter block (single kernel)
-    const int stage_len = kStoreBlock * (nc16 | 1);
+    const int stage_len = FULL ? kStoreBlock * (nc16 | 1) : RB * LB;   // FULL false: U11^-1
     double* pivabs = stage + stage_len;                     // [nmax] |pivot|
     double* redd = pivabs + nmax;                           // [3 * NWAVE]
     int* wsum = reinterpret_cast<int*>(redd + 3 * NWAVE);   // [NWAVE]
@@ -917,7 +927,8 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
         if (s < ns) {
             if (empty) {
                 const int row = N + off + before;
-                if (row < N + nE) { rowsite[row] = s; rowof[s] = row; }
+                if (!FULL) { if (row >= N + nEmpty) s_bad = 1; }
+                else if (row < N + nE) { rowsite[row] = s; rowof[s] = row; }
                 else s_bad = 1;
             } else if (l == 0) {
                 // an empty site of the copied half (real form): no row
@@ -932,11 +943,18 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
         base += tot;
         __syncthreads();
     }
-    if (t == 0 && base != nE) s_bad = 1;
+    if (t == 0 && base != nEmpty) s_bad = 1;
     __syncthreads();
     if (s_bad) {
         if (t == 0) { a.status[w] = 2; atomicMin(a.failed, w); }
         return;
+    }
+    if (!FULL) {
+        // columns nc16..ldm-1 and rows nr16.. of M are read (as zeros) by the
+        // solve kernel
+        const int nz = ldm - nc16, nrz = rup_i(N, RB);
+        for (int idx = t; idx < nrz * nz; idx += RT) M[(size_t)(idx / nz) * ldm + nc16 + idx % nz] = 0.0;
+        for (int idx = t; idx < (nrz - nr16) * ldm; idx += RT) M[(size_t)nr16 * ldm + idx] = 0.0;
     }
     // M is never filled from U up front: the first panel (j0 = 0) reads its
     // operands straight from U (L2-resident, shared by every job) and every
@@ -1051,31 +1069,43 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
             for (int c = 0; c < RB; ++c) Dblk[i * LB + c] = (c == i) ? 1.0 : 0.0;
         }
         __syncthreads();
-        // U11^-1, applied to the empty-site rows, whose panel slice solves
-        // x U11 = a  ->  x = a U11^-1
-        upper_inverse(Dblk, Linv, LB, 0);
-        __syncthreads();
-        const int ntr = m16 / 16;
-        for (int ti = wave; ti < ntr; ti += NWAVE) {
-            const int ra = N + 16 * ti + (lane & 15);
-            f64x4 y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
+        if constexpr (!FULL) {
+            // padding rows N..nr16-1 (phys[r] = r) enter the trailing update
+            // as zero rows; nothing reads their results
+            for (int idx = t; idx < (nr16 - N) * RB; idx += RT) M[(size_t)(N + idx / RB) * ldm + j0 + idx % RB] = 0.0;
+            __syncthreads();
+            upper_inverse(Dblk, stage, LB, 0);
+            unit_lower_inverse(Dblk, Linv, jb, 1);
+            __syncthreads();
+            for (int idx = t; idx < RB * RB; idx += RT)
+                Usave[(size_t)(j0 / RB) * RB * RB + idx] = stage[(idx / RB) * LB + idx % RB];
+        } else {
+            // U11^-1, applied to the empty-site rows, whose panel slice solves
+            // x U11 = a  ->  x = a U11^-1
+            upper_inverse(Dblk, Linv, LB, 0);
+            __syncthreads();
+            const int ntr = m16 / 16;
+            for (int ti = wave; ti < ntr; ti += NWAVE) {
+                const int ra = N + 16 * ti + (lane & 15);
+                f64x4 y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
 #pragma unroll
-            for (int s2 = 0; s2 < RB / 4; ++s2) {
-                const int k = 4 * s2 + (lane >> 4);
-                const double av = j0 == 0 ? u_at(ra, k) : M[(size_t)ra * ldm + j0 + k];
-                y0 = mfma16(av, Linv[k * LB + (lane & 15)], y0);
-                y1 = mfma16(av, Linv[k * LB + 16 + (lane & 15)], y1);
-            }
+                for (int s2 = 0; s2 < RB / 4; ++s2) {
+                    const int k = 4 * s2 + (lane >> 4);
+                    const double av = j0 == 0 ? u_at(ra, k) : M[(size_t)ra * ldm + j0 + k];
+                    y0 = mfma16(av, Linv[k * LB + (lane & 15)], y0);
+                    y1 = mfma16(av, Linv[k * LB + 16 + (lane & 15)], y1);
+                }
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const size_t row = (size_t)(N + 16 * ti + (lane >> 4) + 4 * g) * ldm + j0;
-                M[row + (lane & 15)] = y0[g];
-                M[row + 16 + (lane & 15)] = y1[g];
+                for (int g = 0; g < 4; ++g) {
+                    const size_t row = (size_t)(N + 16 * ti + (lane >> 4) + 4 * g) * ldm + j0;
+                    M[row + (lane & 15)] = y0[g];
+                    M[row + 16 + (lane & 15)] = y1[g];
+                }
             }
+            __syncthreads();
+            unit_lower_inverse(Dblk, Linv, jb, 0);
+            __syncthreads();
         }
-        __syncthreads();
-        unit_lower_inverse(Dblk, Linv, jb, 0);
-        __syncthreads();
         for (int idx = t; idx < RB * RB; idx += RT)
             Lsave[(size_t)(j0 / RB) * RB * RB + idx] = Linv[(idx / RB) * LB + idx % RB];
         const int c0 = j0 + RB;
@@ -1263,6 +1293,12 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
         a.logdet[(size_t)w * 2 + spin] = logdet;
         if (a.write_w) a.stiff[(size_t)w * 2 + spin] = pmin < kStiffTol * pmax;
         if (a.write_w && spin == 0) { a.npend[w] = 0; a.acc_since[w] = 0; }
+    }
+    if constexpr (!FULL) {
+        // logical row c < N holds label phys[c]; W is formed by the solve kernel
+        for (int c = t; c < N; c += RT) jint[1 + c] = phys[c];
+        if (t == 0) jint[0] = 1;
+        return;
     }
     // logical row c < N holds label phys[c]
     for (int c = t; c < N; c += RT) pinv[phys[c]] = c;
@@ -1753,6 +1789,268 @@ k_refresh_solve(RefreshArgs a, int groups) {
     }
 }
 
+// The empty-site rows of W for 256 < N <= 512 (in practice the real form of
+// complex orbitals) from the factors of k_refresh_blocked<FULL = false>, as
+// k_refresh_solve, in blocks of 32 labels with the whole 32x32 inverses.
+//
+// 512 threads per 64 empty sites: two wavefronts share 16 sites, one holds the
+// even and the other the odd 32-label blocks in MFMA accumulators (negated, 16
+// registers a tile pair and half the blocks each, so two wavefronts fit a
+// SIMD).  The wavefront that holds block J forms y_J and hands it to its
+// partner through LDS, a step ahead: the block that comes next is updated
+// first and its y formed before the other updates.  The factors' rows are read
+// as operands straight from memory, 128 bytes a row, two blocks ahead; the
+// wavefronts of a workgroup read the same ones through L1.
+//
+// The single kernel carried the empty rows through memory, read and written
+// once a panel in both solves.  With the products and sums of an element in
+// its order the bits are the same.  Measured in a gradient step of 1000
+// walkers of the complex system of 432 sites (2N = 432), LU and solve: 13.9 ->
+// 9.7 ms.
+template <typename T, int NB>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) k_refresh_solve2(RefreshArgs a, int groups) {
+    constexpr int NH = NB / 2, NTH = 512;
+    __shared__ __align__(16) double sy[2][4][8][64];     // y_J, by parity of J and 16 sites
+    __shared__ __align__(16) double sd[2][RB * RB];      // diagonal inverse, by parity of J
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int b = (int)blockIdx.x;
+    const int job = ((b >> 3) / groups) * 8 + (b & 7);
+    const int grp = (b >> 3) % groups;
+    if (job >= a.njobs) return;
+    const int spin = job & 1;
+    const int ns = a.ns, N = spin ? a.ndn : a.nup, nmax = a.nmax;
+    const int nso = a.ns_out, NO = spin ? a.ndn_out : a.nup_out, cw = a.cplx_out ? 2 : 1;
+    const int nEo = nso - NO;
+    if (grp > 0 && 64 * grp >= nEo) return;
+    const int np = (N + RB - 1) / RB;
+    const double* __restrict__ M = a.ws + (size_t)job * refresh_ws_job(ns, nmax);
+    const int ldm = refresh_ldm(nmax);
+    const double* __restrict__ Lsave = M + (size_t)refresh_nrows(ns) * ldm;
+    const double* __restrict__ Usave = Lsave + (size_t)refresh_npanel(nmax) * RB * RB;
+    const int* __restrict__ jint = reinterpret_cast<const int*>(Usave + (size_t)refresh_npanel(nmax) * RB * RB);
+    const int cnt = a.count_dev ? *a.count_dev : 0;
+    const int w = a.jobs[job >> 1];
+    const int fact = jint[0];
+    if (a.count_dev && job >= 2 * (cnt - a.walker_off)) return;
+    if (fact != 1) return;                               // factorisation rejected (status already set)
+    const int* __restrict__ kap = (spin ? a.kdn : a.kup) + (size_t)w * ns;
+    const double* __restrict__ UT = spin ? a.UTdn : a.UTup;
+    const int t = (int)threadIdx.x, lane = t % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(t / 64);
+    const int q16 = wave & 3, half = wave >> 2;          // group of 16 sites, parity of the blocks held
+    const int kr = lane >> 4, kc = lane & 15;
+
+    int* lab = reinterpret_cast<int*>(lds);              // [NB * 32] logical row -> physical row of M
+    int* wsum = lab + NB * RB;                           // [8]
+    int* esite = wsum + 8;                               // [nso] empty sites in order
+
+    for (int c = t; c < NB * RB; c += NTH) lab[c] = c < N ? jint[1 + c] : c;
+    int base = 0;
+    for (int s0 = 0; s0 < nso; s0 += NTH) {
+        const int s = s0 + t;
+        const bool empty = s < nso && kap[s] == 0;
+        const unsigned long long m = __ballot(empty);
+        const int before = __popcll(m & ((1ull << lane) - 1ull));
+        if (lane == 0) wsum[wave] = __popcll(m);
+        __syncthreads();
+        int off = base, tot = 0;
+        for (int q = 0; q < 8; ++q) {
+            off += q < wave ? wsum[q] : 0;
+            tot += wsum[q];
+        }
+        if (empty) esite[off + before] = s;
+        base += tot;
+        __syncthreads();
+    }
+    const int e = 64 * grp + 16 * q16 + kc;
+    const int site = e < nEo ? esite[e] : -1;
+
+    f64x4 tile[NH][2];                                   // block 2 i + half, its two 16-label tiles
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int c = RB * (2 * i + half) + 16 * h + kr + 4 * g;
+                tile[i][h][g] = (site >= 0 && c < N) ? -UT[(size_t)site * N + c] : 0.0;
+            }
+        }
+    }
+    auto stage = [&](const double* inv, int J) {         // 16 bytes a thread
+        __builtin_amdgcn_global_load_lds(inv + (size_t)J * RB * RB + 2 * t, (lds_void*)(&sd[J & 1][0] + 128 * wave), 16, 0, 0);
+    };
+    // y = (-inv)^T T of this wavefront's block i, number J; lower: of L11^-1,
+    // else of U11^-1 (the 16x16 block beyond the diagonal is zero)
+    auto publish = [&](int i, int J, bool lower) {
+        const double* d = sd[J & 1];
+        f64x4 y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const double tv = s < 4 ? tile[i][0][s & 3] : tile[i][1][s & 3];
+            if (lower || s < 4) y0 = mfma16(-d[(4 * s + kr) * RB + kc], tv, y0);
+            if (!lower || s >= 4) y1 = mfma16(-d[(4 * s + kr) * RB + 16 + kc], tv, y1);
+        }
+        tile[i][0] = y0;
+        tile[i][1] = y1;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            sy[J & 1][q16][g][lane] = y0[g];
+            sy[J & 1][q16][4 + g][lane] = y1[g];
+        }
+    };
+    const double* rp[8];                                 // the factor rows of block J, at this half's columns
+    double va[2][2][8];
+    auto rows = [&](int J) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) rp[s] = M + (size_t)lab[RB * J + 4 * s + kr] * ldm + RB * half + kc;
+    };
+    auto fetch = [&](double (&v)[2][8], int i) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) v[h][s] = rp[s][2 * RB * i + 16 * h];
+        }
+    };
+    double y[8];
+    auto update = [&](const double (&v)[2][8], int i) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) tile[i][h] = mfma16(v[h][s], y[s], tile[i][h]);
+        }
+    };
+    auto take = [&](int J) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) y[s] = sy[J & 1][q16][s][lane];
+    };
+
+    if (np > 0) stage(Usave, 0);
+    __syncthreads();
+    if (half == 0 && np > 0) publish(0, 0, false);
+    // y U1 = b, blocks ascending
+#pragma unroll
+    for (int J = 0; J < NB; ++J) {
+        if (J < np) {
+            const int j = J / 2 + 1;                     // first block of either parity after J (half 1 of an even J: j - 1 too)
+            rows(J);
+            if (j < NH) fetch(va[0], j);
+            if (j + 1 < NH) fetch(va[1], j + 1);
+            if (J + 1 < np) stage(Usave, J + 1);
+            __syncthreads();                             // y_J, the next inverse
+            take(J);
+            if ((J & 1) == 0 && half == 1) {
+                double v[2][8];
+                fetch(v, j - 1);
+                update(v, j - 1);
+                if (J + 1 < np) publish(j - 1, J + 1, false);
+            }
+#pragma unroll
+            for (int i = j; i < NH; ++i) {
+                update(va[(i - j) & 1], i);
+                if (i + 2 < NH) fetch(va[(i - j) & 1], i + 2);
+                __builtin_amdgcn_sched_barrier(0);
+                if ((J & 1) == 1 && i == j && half == 0 && J + 1 < np) publish(i, J + 1, false);
+            }
+        }
+    }
+    // the second solve starts from T_K = -y_K
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+        tile[i][0] = -tile[i][0];
+        tile[i][1] = -tile[i][1];
+    }
+    // every wavefront is past its reads of the first solve's last inverse and y
+    __syncthreads();
+    if (np > 0) stage(Lsave, np - 1);
+    __syncthreads();
+    // x L1 = y, blocks descending
+#pragma unroll
+    for (int J = NB - 1; J >= 0; --J) {
+        if (J < np) {
+            if (J == np - 1 && half == (J & 1)) publish(J / 2, J, true);
+            // blocks before J: i < J / 2, and for odd J the even half's i = J / 2
+            const int j = J / 2 - 1;
+            rows(J);
+            if (j >= 0) fetch(va[0], j);
+            if (j - 1 >= 0) fetch(va[1], j - 1);
+            if (J > 0) stage(Lsave, J - 1);
+            __syncthreads();
+            take(J);
+            if ((J & 1) == 1 && half == 0) {
+                double v[2][8];
+                fetch(v, j + 1);
+                update(v, j + 1);
+                publish(j + 1, J - 1, true);
+            }
+#pragma unroll
+            for (int i = j; i >= 0; --i) {
+                update(va[(j - i) & 1], i);
+                if (i - 2 >= 0) fetch(va[(j - i) & 1], i - 2);
+                __builtin_amdgcn_sched_barrier(0);
+                if ((J & 1) == 0 && i == j && half == 1) publish(i, J - 1, true);
+            }
+        }
+    }
+
+    // ---- W: the solved tiles, one row per empty site; the slot map --------
+    T* __restrict__ Wo = reinterpret_cast<T*>(a.W) +
+                         ((size_t)w * w_stride(nso, a.nup_out, a.ndn_out) + (spin ? w_off_dn(nso, a.nup_out) : 0)) * cw;
+    const int ld = w_ld(nso, NO);
+    int* __restrict__ sl = a.slot + ((size_t)w * 2 + spin) * nso;
+    const int nsa = w_nsa(nso, a.nup_out, a.ndn_out);
+    const int cpend = a.write_w ? 0 : a.npend[w];
+    const int dp = pend_ld(a.delay);
+    const T* gA = reinterpret_cast<const T*>(a.A) + ((size_t)w * 2 + spin) * nsa * dp * cw;
+    const T* gB = reinterpret_cast<const T*>(a.Bm) + ((size_t)w * 2 + spin) * a.nmax_out * dp * cw;
+    double dmax = 0.0, vmax = N > 0 ? 1.0 : 0.0;   // occupied rows: unit rows, exact
+    if (site >= 0) {
+        const int row = a.write_w ? e : max(sl[site], 0);
+#pragma unroll
+        for (int i = 0; i < NH; ++i) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int c = RB * (2 * i + half) + 16 * h + kr + 4 * g;
+                    if (c < N) {
+                        const int l = lab[c];
+                        const int part = l >= NO ? 1 : 0, lo = l - part * NO;
+                        const double v = part ? -tile[i][h][g] : tile[i][h][g];
+                        const size_t at = (size_t)lo * ld + row;
+                        if (a.write_w) {
+                            Wo[at * cw + part] = (T)v;
+                        } else {
+                            double cur = (double)Wo[at * cw + part];
+                            for (int q = 0; q < cpend; ++q) {
+                                const size_t ia = ((size_t)row * dp + q) * cw, ib = ((size_t)lo * dp + q) * cw;
+                                if (cw == 1) {
+                                    cur += (double)gA[ia] * (double)gB[ib];
+                                } else {
+                                    const double ar = gA[ia], ai = gA[ia + 1], br = gB[ib], bi = gB[ib + 1];
+                                    cur += part ? ar * bi + ai * br : ar * br - ai * bi;
+                                }
+                            }
+                            dmax = fmax(dmax, fabs(v - cur));
+                            vmax = fmax(vmax, fabs(v));
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (a.write_w) {
+        const int s_lo = grp == 0 ? 0 : esite[64 * grp];
+        const int s_hi = 64 * (grp + 1) < nEo ? esite[64 * (grp + 1)] : nso;
+        for (int s = s_lo + t; s < s_hi; s += NTH)
+            if (kap[s] != 0) sl[s] = -1;
+        if (t < 64 && 64 * grp + t < nEo) sl[esite[64 * grp + t]] = 64 * grp + t;
+    } else {
+        atomic_max_nonneg2(&a.drift[(size_t)w * 2], dmax);
+        atomic_max_nonneg2(&a.drift[(size_t)w * 2 + 1], vmax);
+    }
+}
+
 // LDS of k_refresh_solve: static row-block buffers plus the dynamic part.
 static size_t solve_static_lds(int nt) { return (size_t)(2 * nt * 256 + 2 * 256) * sizeof(double); }
 static size_t solve_lds_bytes(int ns, int nt) { return (size_t)(nt * 16 + NWAVE + ns) * sizeof(int); }
@@ -1776,11 +2074,11 @@ static hipError_t set_lds_limit(const void* fn, size_t lds) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
-template <typename T, int RPT>
+template <typename T, int RPT, bool FULL = true>
 static hipError_t launch_single(const RefreshArgs& a, size_t lds, hipStream_t s) {
-    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, RPT>), lds);
+    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, RPT, FULL>), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_refresh_blocked<T, RPT>), dim3(a.njobs), dim3(RT), lds, s, a);
+    hipLaunchKernelGGL((k_refresh_blocked<T, RPT, FULL>), dim3(a.njobs), dim3(RT), lds, s, a);
     return hipGetLastError();
 }
 
@@ -1819,6 +2117,26 @@ static int solve_tiles(int ns, int nmax) {
     return NT;
 }
 
+static size_t solve2_lds_bytes(int ns_out, int nb) { return (size_t)(nb * RB + 8 + ns_out) * sizeof(int); }
+
+template <typename T, int NB>
+static hipError_t launch_solve2(const RefreshArgs& a, hipStream_t s) {
+    const int nmin = a.nup_out < a.ndn_out ? a.nup_out : a.ndn_out;
+    const int groups = (a.ns_out - nmin + 63) / 64 > 1 ? (a.ns_out - nmin + 63) / 64 : 1;
+    const size_t lds = solve2_lds_bytes(a.ns_out, NB);
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_refresh_solve2<T, NB>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((k_refresh_solve2<T, NB>), dim3(8 * groups * ((a.njobs + 7) / 8)), dim3(512), lds, s, a, groups);
+    return hipGetLastError();
+}
+
+// 32-label blocks of k_refresh_solve2 for 256 < N <= 512, an even number, or 0.
+static int solve2_blocks(int ns, int nmax) {
+    const int nb = rup_i(refresh_npanel(nmax), 2);
+    return nmax > 256 && nb <= 16 && 48 * 1024 + solve2_lds_bytes(ns, nb) <= 160 * 1024 ? nb : 0;
+}
+
 template <typename T>
 static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t s) {
     const int tiles = solve_tiles(a.ns, a.nmax);
@@ -1843,6 +2161,18 @@ static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t
             case 12: return launch_solve<T, 12>(a, s);
             case 14: return launch_solve<T, 14>(a, s);
             default: return launch_solve<T, 16>(a, s);
+        }
+    }
+    // from 257 to 512 labels two kernels, measured 13.9 against 9.7 ms at 432;
+    // beyond, half the tiles no longer fit a wavefront's registers
+    if (solve2_blocks(a.ns, a.nmax)) {
+        hipError_t e = launch_single<T, 2, false>(a, lds, s);
+        if (e != hipSuccess) return e;
+        switch (solve2_blocks(a.ns, a.nmax)) {
+            case 10: return launch_solve2<T, 10>(a, s);
+            case 12: return launch_solve2<T, 12>(a, s);
+            case 14: return launch_solve2<T, 14>(a, s);
+            default: return launch_solve2<T, 16>(a, s);
         }
     }
     switch (refresh_rows_per_thread(a.nmax)) {

@@ -30,3 +30,15 @@ def test_zero_pivot_is_refused(n, col):
     with nat.DeviceSampler(bonds, Uu, Ud, 2) as ds:
         with pytest.raises(nat.SingularError):
             ds.set_configs(k[0], k[1])
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n_up,n_dn,cplx", [(257, 31, False), (288, 289, False), (320, 321, False),
+                                            (385, 352, False), (449, 448, False), (511, 512, False),
+                                            (40, 512, False), (513, 500, False), (129, 128, True), (144, 145, True), (160, 161, True),
+                                            (225, 3, True), (240, 256, True), (257, 250, True)],
+                         ids=lambda x: str(x))
+def test_refresh_split_over_two_wavefronts(n_up, n_dn, cplx, prec):
+    """257 to 512 labels (twice as many as complex orbitals): edges of its
+    32-label blocks and pairs of blocks, a spin far below, and one beyond."""
+    check_refresh(n_up, n_dn, cplx, prec, 4000 + n_up)
