@@ -936,7 +936,7 @@ __global__ void __launch_bounds__(256) k_grad(ElocArgs a) {
     for (int p = tid; p < CW * P; p += (int)blockDim.x) a.O[(size_t)w * CW * P + p] = acc[p];
 }
 
-// The same sums taken site by site, for up to PM parameters: every site s
+// The same sums taken site by site, for P parameters: every site s
 // holds one electron (label l of the spin at s), so
 //   O_k = sum_s ( Q_k[s, s] + sum_r W[slot(r), l] Q_k[s, r] )
 // over the empty sites r of that spin.  A workgroup takes GW walkers with
@@ -944,22 +944,26 @@ __global__ void __launch_bounds__(256) k_grad(ElocArgs a) {
 // quarter q of walker g.  The GW wavefronts of a quarter walk its sites in
 // the same order, so each Q row is fetched from L2 once per workgroup and
 // served to the other walkers from L1.  Each W element is read once, for all
-// parameters at a time.  Labels and slot maps are staged in LDS (16-bit), so
-// a site costs one memory round trip (its W and Q loads together).
+// parameters at a time.  Labels and slot maps are staged in LDS (16-bit).
+// The loads of 192 sites r go out together, unconditionally (an occupied or
+// missing site reads an entry that is not used), so a site costs one or two
+// memory round trips; behind a branch on r every 64 of them cost one.
+// Bound: the latency of those round trips (the Q rows of four walkers come
+// from L2 once).  432 sites, 1000 complex walkers: 1.65 -> 0.85 ms.
 constexpr int kGradWalkers = 4;   // walkers per workgroup of k_grad_sites
-template <typename T, int PM>
+template <typename T, int P>
 __global__ void __launch_bounds__(1024) k_grad_sites(ElocArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     using A = typename AccT<T>::type;
     constexpr int CW = is_cplx<T>::value ? 2 : 1;   // doubles per value
-    constexpr int GW = kGradWalkers;
+    constexpr int GW = kGradWalkers, RU = 3;
     const int wave = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
     const int g = wave % GW, q = wave / GW;          // walker slot, quarter of the sites
     const int w = (int)blockIdx.x * GW + g;
     const bool live = w < a.nw;                      // every wavefront reaches both barriers
-    const int ns = a.ns, nsp = round_up(ns, 4), P = a.nparams;
-    double* red = reinterpret_cast<double*>(lds);    // [GW][4][PM][CW]
-    int16_t* mk = reinterpret_cast<int16_t*>(red + GW * 4 * PM * CW) + (size_t)g * 4 * nsp;   // kup, kdn, slots
+    const int ns = a.ns, nsp = round_up(ns, 4);
+    double* red = reinterpret_cast<double*>(lds);    // [GW][4][P][CW]
+    int16_t* mk = reinterpret_cast<int16_t*>(red + GW * 4 * P * CW) + (size_t)g * 4 * nsp;   // kup, kdn, slots
     if (live) {
         const int* ku = a.kup + (size_t)w * ns;
         const int* kd = a.kdn + (size_t)w * ns;
@@ -972,9 +976,9 @@ __global__ void __launch_bounds__(1024) k_grad_sites(ElocArgs a) {
         }
     }
     __syncthreads();
-    A part[PM];
+    A part[P];
 #pragma unroll
-    for (int p = 0; p < PM; ++p) part[p] = A(0.0);
+    for (int p = 0; p < P; ++p) part[p] = A(0.0);
     if (live) {
         const int ldu = w_ld(ns, a.nup), ldd = w_ld(ns, a.ndn);
         const T* Wup = reinterpret_cast<const T*>(a.W) + (size_t)w * w_stride(ns, a.nup, a.ndn);
@@ -993,39 +997,48 @@ __global__ void __launch_bounds__(1024) k_grad_sites(ElocArgs a) {
             const A* qs = (up ? Qu : Qd) + (size_t)s * ns;
             if (lane == 0) {
 #pragma unroll
-                for (int p = 0; p < PM; ++p)
-                    if (p < P) part[p] += qs[p * qstride + s];
+                for (int p = 0; p < P; ++p) part[p] += qs[p * qstride + s];
             }
-            for (int r = lane; r < ns; r += 64) {
-                const int e = sl[r];
-                if (e >= 0) {
-                    const A wv = to_acc(wcol[e]);
+            for (int r0 = lane; r0 < ns; r0 += 64 * RU) {
+                A wv[RU], qv[RU][P];
+                bool use[RU];
 #pragma unroll
-                    for (int p = 0; p < PM; ++p)
-                        if (p < P) part[p] += wv * qs[p * qstride + r];
+                for (int i = 0; i < RU; ++i) {
+                    const int r = min(r0 + 64 * i, ns - 1), e = sl[r];
+                    use[i] = r0 + 64 * i < ns && e >= 0;
+                    wv[i] = to_acc(wcol[max(e, 0)]);
+#pragma unroll
+                    for (int p = 0; p < P; ++p) qv[i][p] = qs[p * qstride + r];
+                }
+#pragma unroll
+                for (int i = 0; i < RU; ++i) {
+                    if (use[i]) {
+#pragma unroll
+                        for (int p = 0; p < P; ++p) part[p] += wv[i] * qv[i][p];
+                    }
                 }
             }
         }
     }
 #pragma unroll
-    for (int p = 0; p < PM; ++p) {
+    for (int p = 0; p < P; ++p) {
         double pr = re_of(part[p]), pi = im_of(part[p]);
         for (int o = 32; o > 0; o >>= 1) {
             pr += __shfl_xor(pr, o, 64);
             if constexpr (CW == 2) pi += __shfl_xor(pi, o, 64);
         }
         if (lane == 0) {
-            red[((g * 4 + q) * PM + p) * CW] = pr;
-            if constexpr (CW == 2) red[((g * 4 + q) * PM + p) * CW + 1] = pi;
+            red[((g * 4 + q) * P + p) * CW] = pr;
+            if constexpr (CW == 2) red[((g * 4 + q) * P + p) * CW + 1] = pi;
         }
     }
     __syncthreads();
-    if (live && q == 0 && lane < CW * PM) {
+    if (live && q == 0 && lane < CW * P) {
         const int p = lane / CW, c = lane % CW;
-        if (p < P) {
+        {
             double v = 0.0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v += red[((g * 4 + k) * PM + p) * CW + c];
+            for (int k = 0; k < 4; ++k) v += red[((g * 4 + k) * P + p) * CW + c];
             a.O[(size_t)w * CW * P + CW * p + c] = v;
         }
     }
@@ -1036,10 +1049,15 @@ hipError_t launch_grad_t(const ElocArgs& a, hipStream_t s) {
     constexpr int CW = is_cplx<T>::value ? 2 : 1;
     if (a.nparams <= 4) {
         constexpr int GW = kGradWalkers;
-        const size_t lds = (size_t)GW * 4 * 4 * CW * sizeof(double) +                 // partial sums
+        const size_t lds = (size_t)GW * 4 * a.nparams * CW * sizeof(double) +         // partial sums
                            (size_t)GW * 4 * ((a.ns + 3) / 4 * 4) * sizeof(int16_t);    // maps per walker
-        hipLaunchKernelGGL((k_grad_sites<T, 4>), dim3((unsigned)((a.nw + GW - 1) / GW)), dim3(64 * 4 * GW), lds, s,
-                           a);
+        const dim3 grid((unsigned)((a.nw + GW - 1) / GW)), block(64 * 4 * GW);
+        switch (a.nparams) {
+            case 0: case 1: hipLaunchKernelGGL((k_grad_sites<T, 1>), grid, block, lds, s, a); break;
+            case 2: hipLaunchKernelGGL((k_grad_sites<T, 2>), grid, block, lds, s, a); break;
+            case 3: hipLaunchKernelGGL((k_grad_sites<T, 3>), grid, block, lds, s, a); break;
+            default: hipLaunchKernelGGL((k_grad_sites<T, 4>), grid, block, lds, s, a); break;
+        }
         return hipGetLastError();
     }
     const size_t lds = (size_t)(2 * a.nmax + 2) * sizeof(int) + (size_t)CW * a.nparams * sizeof(double) + 16;
