@@ -61,9 +61,8 @@ __host__ __device__ inline int solve_nt(int nmax) {
     const int nt = (nmax + 15) / 16;
     return nt <= 16 ? (nt + 1) / 2 * 2 : 0;
 }
-// Row stride of M: whole 16 * NT rows for the solve kernel's row loads (up to
-// 512: whole pairs of 32-label blocks).
-__host__ __device__ inline int refresh_ldm(int nmax) { return solve_nt(nmax) ? 16 * solve_nt(nmax) : rup_i(nmax, nmax <= 512 ? 64 : 32); }
+// Row stride of M: whole 16 * NT rows for the solve kernel's row loads.
+__host__ __device__ inline int refresh_ldm(int nmax) { return solve_nt(nmax) ? 16 * solve_nt(nmax) : rup_i(nmax, 32); }
 __host__ __device__ inline int refresh_npanel(int nmax) { return (nmax + RB - 1) / RB; }
 // Work doubles per job: the padded tall matrix, the saved 32x32 inverses of
 // the diagonal blocks of L1 and of U1, then ints: [0] factorisation ok flag,
@@ -1801,6 +1800,9 @@ k_refresh_solve(RefreshArgs a, int groups) {
 // first and its y formed before the other updates.  The factors' rows are read
 // as operands straight from memory, 128 bytes a row, two blocks ahead; the
 // wavefronts of a workgroup read the same ones through L1.
+//
+// With an odd number of blocks the last tile pair reads what follows the rows (in
+// bounds: the inverses lie behind them); it is never a block of y.
 //
 // The single kernel carried the empty rows through memory, read and written
 // once a panel in both solves.  With the products and sums of an element in
