@@ -45,10 +45,10 @@ HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 
 # HBM bytes (FETCH_SIZE + WRITE_SIZE, calibrated against a plain copy) per
-# walker refreshed by the kernel pair k_refresh_blocked + k_refresh_solve, from
-# rocprofv3 --pmc passes over this script's default FP32 run (summaries in
+# walker refreshed by the kernel pair k_lu + k_refresh_solve, from
+# rocprofv3 --pmc passes over a refresh of 8192 walkers at L=12 (summary in
 # profiles/).
-REFRESH_TRAFFIC_BYTES_PER_WALKER = {12: 6_157_947}
+REFRESH_TRAFFIC_BYTES_PER_WALKER = {12: 5_548_823}
 # the same for the FP32 sweep kernel (k_sweep_ib), per walker-sweep (delay 12,
 # L=12, refresh every 216 accepts)
 SWEEP_TRAFFIC_BYTES_PER_WALKER_SWEEP = {12: 10_394}
@@ -341,18 +341,22 @@ def roofline_refresh(r, ns, traffic_per_walker):
     return {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS,
             "traffic": traffic_per_walker * wpl if traffic_per_walker else None,
-            "kernel": "k_refresh_blocked + k_refresh_solve (FP64 pivoted LU of tildeU, then MFMA "
+            "kernel": "k_lu + k_refresh_solve (FP64 pivoted LU of tildeU, then MFMA "
                       "triangular solves for the empty-site rows of W = U tildeU^-1)",
             "units_per_launch": wpl, "launch_ms": r["refresh_ms_per_launch"]}
 
 
 def sweep_kernel_name(ham, s, delay):
-    """The sweep kernel the library runs for this shape: FP32 W streamed from
-    HBM with at most 256 empty-site rows per spin and 1 < delay <= 16 uses
-    the implicit-pending-row kernel, everything else k_sweep."""
+    """The sweep kernel the library runs for this shape: W streamed from HBM
+    with at most 256 empty-site rows per spin uses the implicit-pending-row
+    kernel (FP32 for 1 < delay <= 16, FP64 for any delay up to 16), small
+    clusters with both W in LDS and at most 64 rows, labels and 128 sites
+    k_sweep_w1, everything else k_sweep."""
     rows = [((ham.ns - n) + 3) // 4 * 4 for n in (ham.N_up, ham.N_down)]
     resident = s * sum(r * n for r, n in zip(rows, (ham.N_up, ham.N_down))) <= 64 * 1024
-    if s == 4 and 1 < delay <= 16 and max(rows) <= 256 and not resident:
+    if resident and max(max(rows), ham.N_up, ham.N_down) <= 64 and ham.ns <= 128:
+        return "k_sweep_w1 (one wavefront per walker, W resident in LDS)"
+    if (1 if s == 4 else 0) < delay <= 16 and max(rows) <= 256 and not resident:
         return "k_sweep_ib (exchange step + delayed Sherman-Morrison updates, pending rows implicit)"
     return "k_sweep (exchange step + delayed Sherman-Morrison updates)"
 

@@ -298,8 +298,9 @@ __device__ __forceinline__ void upper_inverse16x2(const double* D, double* Uinv,
 // J's own step on those columns.
 //
 // Bound: the chain of pivots, about 1700 cycles a column (key, maxima, LDS
-// round trip, reciprocal, update), and in the steps the reads of L, which lies
-// beyond L2 for the jobs in flight.  A panel in the registers of four
+// round trip, reciprocal, update), and at N = 216 HBM: 2.4 MB a matrix, 3.9
+// TB/s, most of it L read again by the steps and the panel's slices on their
+// way (the jobs in flight exceed the caches).  A panel in the registers of four
 // wavefronts, with a barrier and an LDS exchange a column, kept the matrix
 // cores waiting for it (64% of the time at N = 96, 42% at 216), and its
 // right-looking update read and wrote every trailing element once a panel.
