@@ -68,10 +68,16 @@ template <typename R> struct real_of<cplx<R>> { using type = R; };
 // site the electron left.
 __host__ __device__ inline int w_ld(int ns, int n) { return (ns - n + 3) / 4 * 4; }
 __host__ __device__ inline size_t w_off_dn(int ns, int nup) { return (size_t)w_ld(ns, nup) * nup; }
-// Pending rank-1 terms in HBM: A as [walker][spin][row < w_nsa][pend_ld],
-// B as [walker][spin][label < nmax][pend_ld], so the terms of one row (or
-// label) are contiguous and 16-byte aligned.
+// Pending rank-1 terms in HBM, per walker and spin: A over the w_nsa rows of W
+// and B over the nmax labels, in planes of 16 bytes a row (or label): plane
+// q / V holds terms q / V * V .. + V - 1 of every row, V = 16 / element size.
+// A kernel moves the planes of the live terms only, as contiguous vectors;
+// with the pend_ld slots of a row side by side, the lines of all of them moved
+// (L=12, FP64, 12 slots: 83 KB a walker at half of them live).
 __host__ __device__ inline int pend_ld(int delay) { return (delay + 3) / 4 * 4; }
+__host__ __device__ inline size_t pend_at(int V, int rows, int row, int q) {
+    return ((size_t)(q / V) * rows + row) * V + q % V;
+}
 // Number of rows of the pending columns A_q (the rows of the taller W).
 __host__ __device__ inline int w_nsa(int ns, int nup, int ndn) {
     const int a = w_ld(ns, nup), b = w_ld(ns, ndn);
@@ -127,8 +133,8 @@ struct SweepArgs {
     int* kdn;
     void* W;                        // [nw][w_stride] empty-site rows, column-major per spin
     int* slot;                      // [nw][2][ns] site -> row of W (-1: occupied)
-    void* A;                        // [nw][2][w_nsa][pend_ld]  pending columns (over rows of W)
-    void* Bm;                       // [nw][2][nmax][pend_ld] pending scaled rows
+    void* A;                        // [nw][2][pend_ld * w_nsa] pending columns (over rows of W), see pend_at
+    void* Bm;                       // [nw][2][pend_ld * nmax] pending scaled rows
     int* npend;                     // [nw] pending count
     int delay;                      // 1 = immediate rank-1 update
     int nmax;                       // max(nup, ndn)

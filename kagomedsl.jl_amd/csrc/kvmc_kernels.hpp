@@ -207,40 +207,42 @@ __device__ __forceinline__ void append_terms(const T* __restrict__ Wup, const T*
     }
 }
 
-// Pending terms between HBM ([spin][row][dp], one row's terms contiguous)
-// and LDS ([spin][q][row], one term's column contiguous); only the c live
-// terms move.  One thread per row of A or label of B.
+// Pending terms between HBM (planes, pend_at) and LDS ([spin][q][row], one
+// term's column contiguous); only the c live terms move.  One thread per row
+// of A or label of B.
 template <typename T>
 __device__ __forceinline__ void pend_load(T* s_A, T* s_B, const T* gA, const T* gB, int nsa,
                                           int nmax, int delay, int dp, int c) {
+    constexpr int V = 16 / (int)sizeof(T);
     for (int t = (int)threadIdx.x; t < 2 * nsa; t += (int)blockDim.x) {
-        const int sp = t >= nsa ? 1 : 0;
-        T* d = s_A + sp * delay * nsa + (t - sp * nsa);
-        const T* g = gA + (size_t)t * dp;
-        for (int q = 0; q < c; ++q) d[q * nsa] = g[q];
+        const int sp = t >= nsa ? 1 : 0, row = t - sp * nsa;
+        T* d = s_A + sp * delay * nsa + row;
+        const T* g = gA + (size_t)sp * nsa * dp;
+        for (int q = 0; q < c; ++q) d[q * nsa] = g[pend_at(V, nsa, row, q)];
     }
     for (int t = (int)threadIdx.x; t < 2 * nmax; t += (int)blockDim.x) {
-        const int sp = t >= nmax ? 1 : 0;
-        T* d = s_B + sp * delay * nmax + (t - sp * nmax);
-        const T* g = gB + (size_t)t * dp;
-        for (int q = 0; q < c; ++q) d[q * nmax] = g[q];
+        const int sp = t >= nmax ? 1 : 0, l = t - sp * nmax;
+        T* d = s_B + sp * delay * nmax + l;
+        const T* g = gB + (size_t)sp * nmax * dp;
+        for (int q = 0; q < c; ++q) d[q * nmax] = g[pend_at(V, nmax, l, q)];
     }
 }
 
 template <typename T>
 __device__ __forceinline__ void pend_store(const T* s_A, const T* s_B, T* gA, T* gB, int nsa,
                                            int nmax, int delay, int dp, int c) {
+    constexpr int V = 16 / (int)sizeof(T);
     for (int t = (int)threadIdx.x; t < 2 * nsa; t += (int)blockDim.x) {
-        const int sp = t >= nsa ? 1 : 0;
-        const T* d = s_A + sp * delay * nsa + (t - sp * nsa);
-        T* g = gA + (size_t)t * dp;
-        for (int q = 0; q < c; ++q) g[q] = d[q * nsa];
+        const int sp = t >= nsa ? 1 : 0, row = t - sp * nsa;
+        const T* d = s_A + sp * delay * nsa + row;
+        T* g = gA + (size_t)sp * nsa * dp;
+        for (int q = 0; q < c; ++q) g[pend_at(V, nsa, row, q)] = d[q * nsa];
     }
     for (int t = (int)threadIdx.x; t < 2 * nmax; t += (int)blockDim.x) {
-        const int sp = t >= nmax ? 1 : 0;
-        const T* d = s_B + sp * delay * nmax + (t - sp * nmax);
-        T* g = gB + (size_t)t * dp;
-        for (int q = 0; q < c; ++q) g[q] = d[q * nmax];
+        const int sp = t >= nmax ? 1 : 0, l = t - sp * nmax;
+        const T* d = s_B + sp * delay * nmax + l;
+        T* g = gB + (size_t)sp * nmax * dp;
+        for (int q = 0; q < c; ++q) g[pend_at(V, nmax, l, q)] = d[q * nmax];
     }
 }
 
@@ -631,40 +633,31 @@ hipError_t launch_flush_t(const SweepArgs& a, int nw, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // Local energy (getOL, src/Hamiltonian.jl:762-778 with spinInteraction!
-// :636-672 and SzInteraction! :593-604): one wavefront per walker, lanes
-// stride over the bond list, FP64 accumulation, shuffle reduction.  The
-// reference keeps the real part; complex W also yields the imaginary part
-// (needed by the energy gradient of a complex wave function).
+// :636-672 and SzInteraction! :593-604).  The reference keeps the real part;
+// complex W also yields the imaginary part (needed by the energy gradient of
+// a complex wave function).
 // ---------------------------------------------------------------------------
-// The pending terms' part of W_cur[K][l], added to v: the c terms of row K
-// and of label l are contiguous (pend_ld apart per row).
+// The pending terms' part of W_cur[K][l], added to v: terms of one spin in
+// planes (pend_at) of nsa rows and nmax labels.
 template <typename T>
-__device__ __forceinline__ typename AccT<T>::type w_terms(typename AccT<T>::type v, const T* gA, const T* gB,
-                                                          int dp, int K, int l, int c) {
-    const T* ra = gA + (size_t)K * dp;
-    const T* rb = gB + (size_t)l * dp;
+__device__ __forceinline__ typename AccT<T>::type w_terms(typename AccT<T>::type v, const T* A, const T* B,
+                                                          int nsa, int nmax, int K, int l, int c) {
+    constexpr int V = 16 / (int)sizeof(T);
     if constexpr (!is_cplx<T>::value) {
         // real: the terms as 16-byte vectors
-        constexpr int NV = 16 / (int)sizeof(T);
-        using VT = typename VecT<T, NV>::type;
-        for (int q0 = 0; q0 < c; q0 += NV) {
-            const VT x = *reinterpret_cast<const VT*>(ra + q0);
-            const VT y = *reinterpret_cast<const VT*>(rb + q0);
+        using VT = typename VecT<T, V>::type;
+        const VT* ra = reinterpret_cast<const VT*>(A) + K;
+        const VT* rb = reinterpret_cast<const VT*>(B) + l;
+        for (int q0 = 0; q0 < c; q0 += V, ra += nsa, rb += nmax) {
+            const VT x = *ra, y = *rb;
 #pragma unroll
-            for (int u = 0; u < NV; ++u)
+            for (int u = 0; u < V; ++u)
                 if (q0 + u < c) v += (double)(x[u] * y[u]);
         }
     } else {
-        for (int q = 0; q < c; ++q) v += to_acc(ra[q] * rb[q]);
+        for (int q = 0; q < c; ++q) v += to_acc(A[pend_at(V, nsa, K, q)] * B[pend_at(V, nmax, l, q)]);
     }
     return v;
-}
-
-// W_cur[K][l]: the flushed W0 (label-major, row stride ld) plus the terms.
-template <typename T>
-__device__ __forceinline__ typename AccT<T>::type w_elem(const T* W0, const T* gA, const T* gB, int ld, int dp,
-                                                         int K, int l, int c) {
-    return w_terms<T>(to_acc(W0[(size_t)l * ld + K]), gA, gB, dp, K, l, c);
 }
 
 // off -= 1/2 x y for the exchange term (real part), offi likewise (imaginary).
@@ -675,6 +668,8 @@ __device__ __forceinline__ void exch_acc(double& off, double& offi, cf64 x, cf64
     offi += -0.5 * p.im;
 }
 
+// W without pending terms: one wavefront per walker, lanes stride over the
+// bond list, FP64 accumulation, shuffle reduction.
 // STAGE: each wavefront first copies its walker's labels and row maps into
 // LDS (16-bit, coalesced), so the bond loop goes to memory only for W.
 template <typename T, bool STAGE>
@@ -683,7 +678,7 @@ __global__ void __launch_bounds__(256) k_eloc(ElocArgs a) {
     const int wave = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64;
     const int w = (int)blockIdx.x * ((int)blockDim.x / 64) + wave;
     if (w >= a.nw) return;   // no block-wide barrier below: each wavefront works alone
-    const int ns = a.ns, nmax = a.nmax, nsp = round_up(ns, 4);
+    const int ns = a.ns, nsp = round_up(ns, 4);
     const int ldu = w_ld(ns, a.nup), ldd = w_ld(ns, a.ndn);
     const T* Wup = reinterpret_cast<const T*>(a.W) + (size_t)w * w_stride(ns, a.nup, a.ndn);
     const T* Wdn = Wup + w_off_dn(ns, a.nup);
@@ -711,13 +706,6 @@ __global__ void __launch_bounds__(256) k_eloc(ElocArgs a) {
     auto kd = [&](int x) -> int { return STAGE ? (int)skd[x] : gkd[x]; };
     auto su = [&](int x) -> int { return STAGE ? (int)ssu[x] : gsu[x]; };
     auto sd = [&](int x) -> int { return STAGE ? (int)ssd[x] : gsd[x]; };
-    const int c = a.npend[w];
-    const int nsa = w_nsa(ns, a.nup, a.ndn);
-    const int dp = pend_ld(a.delay);
-    const T* gAu = reinterpret_cast<const T*>(a.A) + (size_t)w * 2 * nsa * dp;
-    const T* gAd = gAu + (size_t)nsa * dp;
-    const T* gBu = reinterpret_cast<const T*>(a.Bm) + (size_t)w * 2 * nmax * dp;
-    const T* gBd = gBu + (size_t)nmax * dp;
     double diag = 0.0, off = 0.0, offi = 0.0;
     unsigned long long nap = 0;
 #pragma unroll 2
@@ -729,11 +717,11 @@ __global__ void __launch_bounds__(256) k_eloc(ElocArgs a) {
         const bool t2 = iu != 0 && jd != 0;   // S-_i S+_j
         // the target sites are empty for the moving spin (no site holds both)
         if (t1)
-            exch_acc(off, offi, w_elem(Wup, gAu, gBu, ldu, dp, max(su(i), 0), ju - 1, c),
-                     w_elem(Wdn, gAd, gBd, ldd, dp, max(sd(j), 0), id - 1, c));
+            exch_acc(off, offi, to_acc(Wup[(size_t)(ju - 1) * ldu + max(su(i), 0)]),
+                     to_acc(Wdn[(size_t)(id - 1) * ldd + max(sd(j), 0)]));
         if (t2)
-            exch_acc(off, offi, w_elem(Wup, gAu, gBu, ldu, dp, max(su(j), 0), iu - 1, c),
-                     w_elem(Wdn, gAd, gBd, ldd, dp, max(sd(i), 0), jd - 1, c));
+            exch_acc(off, offi, to_acc(Wup[(size_t)(iu - 1) * ldu + max(su(j), 0)]),
+                     to_acc(Wdn[(size_t)(jd - 1) * ldd + max(sd(i), 0)]));
         nap += (iu != 0 && jd != 0) || (ju != 0 && id != 0);
         const double szi = iu != 0 ? 0.5 : -0.5, szj = ju != 0 ? 0.5 : -0.5;
         diag += szi * szj;
@@ -751,11 +739,20 @@ __global__ void __launch_bounds__(256) k_eloc(ElocArgs a) {
     }
 }
 
+// Copies the first n 16-byte vectors of each of one or two spins' terms,
+// `stride` vectors apart: the live planes.
+__device__ __forceinline__ void stage_planes(f32x4* d, const f32x4* g, int n, int stride, int spins) {
+#pragma unroll 4
+    for (int t = (int)threadIdx.x; t < spins * n; t += (int)blockDim.x) {
+        const int o = t < n ? t : t - n + stride;
+        d[o] = g[o];
+    }
+}
+
 // FP32 with delayed updates: one workgroup per walker.  The labels, row
-// maps and the walker's pending terms (A as [spin][row][dp], B as
-// [spin][label][dp], both contiguous in HBM) are copied to LDS once, with
-// 16-byte loads, so the bond loop gathers only W from memory; the 256 lanes
-// split the bonds and a block reduction forms E_L.
+// maps and the live planes of the walker's pending terms are copied to LDS
+// once, with 16-byte loads, so the bond loop gathers only W from memory; the
+// 256 lanes split the bonds and a block reduction forms E_L.
 template <typename T>
 size_t eloc_wg_lds(const ElocArgs& a) {
     const size_t nsp = (size_t)(a.ns + 3) / 4 * 4, dp = (size_t)pend_ld(a.delay);
@@ -767,6 +764,7 @@ template <typename T>
 __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int w = (int)blockIdx.x;
+    const int c = a.npend[w];
     const int ns = a.ns, nmax = a.nmax, nsp = round_up(ns, 4);
     const int nsa = w_nsa(ns, a.nup, a.ndn), dp = pend_ld(a.delay);
     const int ldu = w_ld(ns, a.nup), ldd = w_ld(ns, a.ndn);
@@ -776,9 +774,9 @@ __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
     int16_t* skd = sku + nsp;
     int16_t* ssu = skd + nsp;
     int16_t* ssd = ssu + nsp;
-    T* sAu = reinterpret_cast<T*>(ssd + nsp);             // [2][nsa][dp] (8 nsp bytes: 16-byte aligned)
+    T* sAu = reinterpret_cast<T*>(ssd + nsp);             // [2][nsa dp] in planes (8 nsp bytes: 16-byte aligned)
     T* sAd = sAu + (size_t)nsa * dp;
-    T* sBu = sAu + (size_t)2 * nsa * dp;                  // [2][nmax][dp]
+    T* sBu = sAu + (size_t)2 * nsa * dp;                  // [2][nmax dp]
     T* sBd = sBu + (size_t)nmax * dp;
     double* red = reinterpret_cast<double*>(sBu + (size_t)2 * nmax * dp);
     const int t0 = (int)threadIdx.x, bd = (int)blockDim.x;
@@ -791,18 +789,13 @@ __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
         ssu[t] = (int16_t)a.slot[(size_t)w * 2 * ns + t];
         ssd[t] = (int16_t)a.slot[(size_t)w * 2 * ns + ns + t];
     }
-    const int c = a.npend[w];
     if (c > 0) {
-        // dp is a multiple of 4 elements: whole 16-byte vectors
-        const size_t na = 2 * (size_t)nsa * dp * sizeof(T) / 16, nbv = 2 * (size_t)nmax * dp * sizeof(T) / 16;
+        constexpr int V = 16 / (int)sizeof(T);
+        const int nv = (c + V - 1) / V, rv = dp / V;
         const f32x4* gA = reinterpret_cast<const f32x4*>(reinterpret_cast<const T*>(a.A) + (size_t)w * 2 * nsa * dp);
         const f32x4* gB = reinterpret_cast<const f32x4*>(reinterpret_cast<const T*>(a.Bm) + (size_t)w * 2 * nmax * dp);
-        f32x4* dA = reinterpret_cast<f32x4*>(sAu);
-        f32x4* dB = reinterpret_cast<f32x4*>(sBu);
-#pragma unroll 4
-        for (size_t t = t0; t < na; t += bd) dA[t] = gA[t];
-#pragma unroll 4
-        for (size_t t = t0; t < nbv; t += bd) dB[t] = gB[t];
+        stage_planes(reinterpret_cast<f32x4*>(sAu), gA, nsa * nv, nsa * rv, 2);
+        stage_planes(reinterpret_cast<f32x4*>(sBu), gB, nmax * nv, nmax * rv, 2);
     }
     __syncthreads();
     double diag = 0.0, off = 0.0, offi = 0.0, nap = 0.0;
@@ -840,8 +833,8 @@ __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
 #pragma unroll
         for (int u = 0; u < BPT; ++u) {
             if (mv[u])
-                exch_acc(off, offi, w_terms(to_acc(w0u[u]), sAu, sBu, dp, Ku[u], Lu[u], c),
-                         w_terms(to_acc(w0d[u]), sAd, sBd, dp, Kd[u], Ld[u], c));
+                exch_acc(off, offi, w_terms(to_acc(w0u[u]), sAu, sBu, nsa, nmax, Ku[u], Lu[u], c),
+                         w_terms(to_acc(w0d[u]), sAd, sBd, nsa, nmax, Kd[u], Ld[u], c));
         }
     }
     const double v = block_sum_double(diag + off, red);
@@ -855,8 +848,133 @@ __global__ void __launch_bounds__(256) k_eloc_wg(ElocArgs a) {
     }
 }
 
-// FP32 W with delayed updates and its pending terms within 64 KiB of LDS:
-// one workgroup per walker; otherwise one wavefront per walker.
+// Pending terms of both spins beyond 64 KiB, and FP64 W (terms asked for, or
+// kept by the handle for immediate updates): as k_eloc_wg, but with the terms
+// of one spin at a time in LDS.  Both spins' FP64 terms (83 KB at 216 rows and
+// 12 slots) would leave one workgroup per CU.  Bound by HBM: a line per W
+// element and the live planes, 4.6 TB/s where every slot was read.
+// One wavefront per walker that gathered its terms from memory (k_eloc, before)
+// and here, us per launch: 216 rows, 8192 walkers, 12 slots, 495 and 233; 150
+// rows, 4096, 120 and 69; complex 216 rows, 1024, 99 and 35.
+// BPT bonds a thread and pass: 4 by 256 threads, or 2 by 512 where the LDS
+// allows fewer than four workgroups per CU (us at 512 and 256 threads: 216 rows
+// at 12 slots 233, 245, at 8 slots 180, 177; complex 150 rows 29, 32, 96 rows
+// 39, 33).
+template <typename T>
+size_t eloc_spin_lds(const ElocArgs& a) {
+    const size_t nsp = (size_t)(a.ns + 3) / 4 * 4, dp = (size_t)pend_ld(a.delay);
+    return 8 * nsp + ((size_t)w_nsa(a.ns, a.nup, a.ndn) + (size_t)a.nmax) * dp * sizeof(T) + 32 * sizeof(double);
+}
+
+template <typename T, int BPT>
+__global__ void __launch_bounds__(1024 / BPT) k_eloc_spin(ElocArgs a) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    using A = typename AccT<T>::type;
+    const int w = (int)blockIdx.x;
+    const int ns = a.ns, nmax = a.nmax, nsp = round_up(ns, 4);
+    const int nsa = w_nsa(ns, a.nup, a.ndn), dp = pend_ld(a.delay);
+    const int ldu = w_ld(ns, a.nup), ldd = w_ld(ns, a.ndn);
+    const T* Wup = reinterpret_cast<const T*>(a.W) + (size_t)w * w_stride(ns, a.nup, a.ndn);
+    const T* Wdn = Wup + w_off_dn(ns, a.nup);
+    int16_t* sku = reinterpret_cast<int16_t*>(lds);
+    int16_t* skd = sku + nsp;
+    int16_t* ssu = skd + nsp;
+    int16_t* ssd = ssu + nsp;
+    T* sA = reinterpret_cast<T*>(ssd + nsp);              // [nsa dp] in planes (8 nsp bytes: 16-byte aligned)
+    T* sB = sA + (size_t)nsa * dp;                        // [nmax dp]
+    double* red = reinterpret_cast<double*>(sB + (size_t)nmax * dp);
+    const int t0 = (int)threadIdx.x, bd = (int)blockDim.x;
+    const int c = a.npend[w];
+#pragma unroll 2
+    for (int t = t0; t < ns; t += bd) {
+        sku[t] = (int16_t)a.kup[(size_t)w * ns + t];
+        skd[t] = (int16_t)a.kdn[(size_t)w * ns + t];
+        ssu[t] = (int16_t)a.slot[(size_t)w * 2 * ns + t];
+        ssd[t] = (int16_t)a.slot[(size_t)w * 2 * ns + ns + t];
+    }
+    constexpr int V = 16 / (int)sizeof(T);
+    const int nv = (c + V - 1) / V, rv = dp / V;          // planes: live, of a spin
+    const f32x4* gA = reinterpret_cast<const f32x4*>(reinterpret_cast<const T*>(a.A) + (size_t)w * 2 * nsa * dp);
+    const f32x4* gB = reinterpret_cast<const f32x4*>(reinterpret_cast<const T*>(a.Bm) + (size_t)w * 2 * nmax * dp);
+    __syncthreads();
+    double diag = 0.0, off = 0.0, offi = 0.0, nap = 0.0;
+    // as in k_eloc_wg: all of a thread's W gathers before any is used
+    for (int base = 0; base < a.nb; base += BPT * bd) {
+        const int b0 = base + t0;
+        int Ku[BPT], Lu[BPT], Kd[BPT], Ld[BPT];
+        bool mv[BPT];
+        T w0u[BPT], w0d[BPT];
+#pragma unroll
+        for (int u = 0; u < BPT; ++u) {
+            const int b = b0 + u * bd;
+            const bool in = b < a.nb;
+            const int2 bb = in ? a.bonds[b] : make_int2(0, 0);
+            const int i = bb.x, j = bb.y;
+            const int iu = sku[i], ju = sku[j], id = skd[i], jd = skd[j];
+            const bool t1 = ju != 0 && id != 0, t2 = iu != 0 && jd != 0;
+            mv[u] = in && (t1 || t2);
+            Lu[u] = mv[u] ? (t1 ? ju : iu) - 1 : 0;
+            Ku[u] = mv[u] ? max((int)(t1 ? ssu[i] : ssu[j]), 0) : 0;
+            Ld[u] = mv[u] ? (t1 ? id : jd) - 1 : 0;
+            Kd[u] = mv[u] ? max((int)(t1 ? ssd[j] : ssd[i]), 0) : 0;
+            w0u[u] = Wup[(size_t)Lu[u] * ldu + Ku[u]];
+            w0d[u] = Wdn[(size_t)Ld[u] * ldd + Kd[u]];
+            if (in) {
+                nap += (t1 || t2) ? 1.0 : 0.0;
+                const double szi = iu != 0 ? 0.5 : -0.5, szj = ju != 0 ? 0.5 : -0.5;
+                diag += szi * szj;
+            }
+        }
+        A xu[BPT], xd[BPT];
+#pragma unroll
+        for (int u = 0; u < BPT; ++u) { xu[u] = to_acc(w0u[u]); xd[u] = to_acc(w0d[u]); }
+        if (c > 0) {
+            stage_planes(reinterpret_cast<f32x4*>(sA), gA, nsa * nv, 0, 1);
+            stage_planes(reinterpret_cast<f32x4*>(sB), gB, nmax * nv, 0, 1);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < BPT; ++u)
+                if (mv[u]) xu[u] = w_terms(xu[u], sA, sB, nsa, nmax, Ku[u], Lu[u], c);
+            __syncthreads();
+            stage_planes(reinterpret_cast<f32x4*>(sA), gA + (size_t)nsa * rv, nsa * nv, 0, 1);
+            stage_planes(reinterpret_cast<f32x4*>(sB), gB + (size_t)nmax * rv, nmax * nv, 0, 1);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < BPT; ++u)
+                if (mv[u]) xd[u] = w_terms(xd[u], sA, sB, nsa, nmax, Kd[u], Ld[u], c);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < BPT; ++u)
+            if (mv[u]) exch_acc(off, offi, xu[u], xd[u]);
+    }
+    const double v = block_sum_double(diag + off, red);
+    const double napt = block_sum_double(nap, red + 8);
+    double vi = 0.0;
+    if constexpr (is_cplx<T>::value) vi = block_sum_double(offi, red + 16);
+    if (t0 == 0) {
+        a.eloc[w] = v;
+        if (is_cplx<T>::value && a.eloc_im) a.eloc_im[w] = vi;
+        a.nap[w] = (int)napt;
+    }
+}
+
+template <typename T, int BPT>
+hipError_t launch_eloc_spin(const ElocArgs& a, size_t lds, hipStream_t s) {
+    if (lds > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_eloc_spin<T, BPT>),
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_eloc_spin<T, BPT>), dim3(a.nw), dim3(1024 / BPT), lds, s, a);
+    return hipGetLastError();
+}
+
+// Delayed updates: one workgroup per walker, W in FP32 (WG) with the terms of
+// both spins in LDS while they take at most 64 KiB of it, else with one
+// spin's at a time (at most about half of what the sweep kernels keep in LDS,
+// so it fits wherever they run).  Without pending terms: one wavefront per
+// walker.
 template <typename T, bool WG>
 hipError_t launch_eloc_t(const ElocArgs& a, hipStream_t s) {
     if constexpr (WG) {
@@ -865,6 +983,10 @@ hipError_t launch_eloc_t(const ElocArgs& a, hipStream_t s) {
             return hipGetLastError();
         }
     }
+    const size_t lds_spin = eloc_spin_lds<T>(a);
+    if (a.delay > 1 && lds_spin <= 160 * 1024)
+        return lds_spin > 40 * 1024 ? launch_eloc_spin<T, 2>(a, lds_spin, s) : launch_eloc_spin<T, 4>(a, lds_spin, s);
+    // no terms pending (beyond 160 KiB the sweep kernels refuse the delay)
     dim3 grid((a.nw + 3) / 4), block(256);
     const size_t lds = (size_t)4 * 4 * ((a.ns + 3) / 4 * 4) * sizeof(int16_t);   // 4 wavefronts x 4 arrays
     if (lds <= 64 * 1024) hipLaunchKernelGGL((k_eloc<T, true>), grid, block, lds, s, a);

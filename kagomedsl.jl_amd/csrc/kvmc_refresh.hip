@@ -1427,7 +1427,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
     double* xb = stage;                              // [SB][xs]
     const int nsa = w_nsa(nso, a.nup_out, a.ndn_out);
     const int cpend = a.write_w ? 0 : a.npend[w];
-    const int dp = pend_ld(a.delay);
+    const int dp = pend_ld(a.delay), V = 16 / (cw * (int)sizeof(T));
     const T* gA = reinterpret_cast<const T*>(a.A) + ((size_t)w * 2 + spin) * nsa * dp * cw;
     const T* gB = reinterpret_cast<const T*>(a.Bm) + ((size_t)w * 2 + spin) * a.nmax_out * dp * cw;
     double dmax = 0.0, vmax = N > 0 ? 1.0 : 0.0;   // occupied rows: unit rows, exact
@@ -1477,7 +1477,7 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
             } else {
                 double cur = (double)Wo[at * cw + part];
                 for (int c = 0; c < cpend; ++c) {
-                    const size_t ia = ((size_t)row * dp + c) * cw, ib = ((size_t)lo * dp + c) * cw;
+                    const size_t ia = pend_at(V, nsa, row, c) * cw, ib = pend_at(V, a.nmax_out, lo, c) * cw;
                     if (cw == 1) {
                         cur += (double)gA[ia] * (double)gB[ib];
                     } else {   // component `part` of the complex product
@@ -1741,7 +1741,7 @@ k_refresh_solve(RefreshArgs a, int groups) {
     int* __restrict__ sl = a.slot + ((size_t)w * 2 + spin) * nso;
     const int nsa = w_nsa(nso, a.nup_out, a.ndn_out);
     const int cpend = a.write_w ? 0 : a.npend[w];
-    const int dp = pend_ld(a.delay);
+    const int dp = pend_ld(a.delay), V = 16 / (cw * (int)sizeof(T));
     const T* gA = reinterpret_cast<const T*>(a.A) + ((size_t)w * 2 + spin) * nsa * dp * cw;
     const T* gB = reinterpret_cast<const T*>(a.Bm) + ((size_t)w * 2 + spin) * a.nmax_out * dp * cw;
     double dmax = 0.0, vmax = N > 0 ? 1.0 : 0.0;   // occupied rows: unit rows, exact
@@ -1763,7 +1763,7 @@ k_refresh_solve(RefreshArgs a, int groups) {
                     } else {
                         double cur = (double)Wo[at * cw + part];
                         for (int q = 0; q < cpend; ++q) {
-                            const size_t ia = ((size_t)row * dp + q) * cw, ib = ((size_t)lo * dp + q) * cw;
+                            const size_t ia = pend_at(V, nsa, row, q) * cw, ib = pend_at(V, a.nmax_out, lo, q) * cw;
                             if (cw == 1) {
                                 cur += (double)gA[ia] * (double)gB[ib];
                             } else {
@@ -2003,7 +2003,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) k
     int* __restrict__ sl = a.slot + ((size_t)w * 2 + spin) * nso;
     const int nsa = w_nsa(nso, a.nup_out, a.ndn_out);
     const int cpend = a.write_w ? 0 : a.npend[w];
-    const int dp = pend_ld(a.delay);
+    const int dp = pend_ld(a.delay), V = 16 / (cw * (int)sizeof(T));
     const T* gA = reinterpret_cast<const T*>(a.A) + ((size_t)w * 2 + spin) * nsa * dp * cw;
     const T* gB = reinterpret_cast<const T*>(a.Bm) + ((size_t)w * 2 + spin) * a.nmax_out * dp * cw;
     double dmax = 0.0, vmax = N > 0 ? 1.0 : 0.0;   // occupied rows: unit rows, exact
@@ -2026,7 +2026,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) k
                         } else {
                             double cur = (double)Wo[at * cw + part];
                             for (int q = 0; q < cpend; ++q) {
-                                const size_t ia = ((size_t)row * dp + q) * cw, ib = ((size_t)lo * dp + q) * cw;
+                                const size_t ia = pend_at(V, nsa, row, q) * cw, ib = pend_at(V, a.nmax_out, lo, q) * cw;
                                 if (cw == 1) {
                                     cur += (double)gA[ia] * (double)gB[ib];
                                 } else {

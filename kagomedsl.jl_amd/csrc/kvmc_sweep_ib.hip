@@ -45,11 +45,11 @@
 // updates asked for, 74.1 -> 7.0 ms (delay 12 inside).  4096 walkers at 96
 // rows, FP64: 2.56 -> 0.68 ms; 2048 at 96 rows, complex FP64: 4.37 -> 1.38 ms.
 //
-// Between launches the pending terms are kept in the layout of k_sweep (A as
-// [row][term], B as [label][term]) with A = At and B = g, so the local
-// energy, the flush kernel, get_w and the refresh drift check read them
-// unchanged; the rows g are gathered once at launch exit.  The term rows and
-// labels (K_r, l_r) are kept beside them for the next launch.
+// Between launches the pending terms are kept in the layout of k_sweep
+// (pend_at) with A = At and B = g, so the local energy, the flush kernel,
+// get_w and the refresh drift check read them unchanged; the rows g are
+// gathered once at launch exit.  The term rows and labels (K_r, l_r) are kept
+// beside them for the next launch.
 #include "kvmc_kernels.hpp"
 
 namespace kvmc {
@@ -303,7 +303,7 @@ k_sweep_ib(SweepArgs a) {
         s_slu[t] = (int16_t)slot_g[t];
         s_sld[t] = (int16_t)slot_g[ns + t];
     }
-    constexpr int NVC = (DMAX + V - 1) / V;   // 16-byte vectors per row of terms (dp a multiple of 4 elements)
+    constexpr int NVC = (DMAX + V - 1) / V;   // planes of terms (dp a multiple of 4 elements)
     if (c > 0) {
         const T* gA = reinterpret_cast<const T*>(a.A) + (size_t)w * 2 * nsa * dp;
         const int* pt = a.pterm + (size_t)w * 2 * kMaxDelay * 2;
@@ -311,11 +311,11 @@ k_sweep_ib(SweepArgs a) {
         for (int t = tid; t < 2 * nsa; t += bd) {
             const int sp = t >= nsa ? 1 : 0;
             T* d = s_At + sp * delay * nsa + (t - sp * nsa);
-            const VT* g = reinterpret_cast<const VT*>(gA + (size_t)t * dp);
+            const VT* g = reinterpret_cast<const VT*>(gA + (size_t)sp * nsa * dp) + (t - sp * nsa);
             VT v[NVC];
 #pragma unroll
             for (int p = 0; p < NVC; ++p)
-                if (V * p < c) v[p] = g[p];
+                if (V * p < c) v[p] = g[p * nsa];
 #pragma unroll
             for (int p = 0; p < NVC; ++p) {
                 const T* e = reinterpret_cast<const T*>(&v[p]);
@@ -611,7 +611,7 @@ k_sweep_ib(SweepArgs a) {
         for (int t = tid; t < 2 * nsa; t += bd) {
             const int sp = t >= nsa ? 1 : 0;
             const T* d = s_At + sp * delay * nsa + (t - sp * nsa);
-            VT* g = reinterpret_cast<VT*>(gA + (size_t)t * dp);
+            VT* g = reinterpret_cast<VT*>(gA + (size_t)sp * nsa * dp) + (t - sp * nsa);
 #pragma unroll
             for (int p = 0; p < NVC; ++p) {
                 if (V * p < c) {
@@ -619,7 +619,7 @@ k_sweep_ib(SweepArgs a) {
                     T* e = reinterpret_cast<T*>(&v);
 #pragma unroll
                     for (int u = 0; u < V; ++u) e[u] = V * p + u < c ? d[(V * p + u) * nsa] : T(0);
-                    g[p] = v;
+                    g[p * nsa] = v;
                 }
             }
         }
@@ -632,10 +632,10 @@ k_sweep_ib(SweepArgs a) {
 #pragma unroll
             for (int q = 0; q < V * NVC; ++q)
                 v[q] = q < c ? col[s_K[sp * kMaxDelay + q]] - (l == s_L[sp * kMaxDelay + q] ? T(1) : T(0)) : T(0);
-            VT* g = reinterpret_cast<VT*>(gB + (size_t)t * dp);
+            VT* g = reinterpret_cast<VT*>(gB + (size_t)sp * nmax * dp) + l;
 #pragma unroll
             for (int p = 0; p < NVC; ++p)
-                if (V * p < c) g[p] = *reinterpret_cast<const VT*>(&v[V * p]);
+                if (V * p < c) g[p * nmax] = *reinterpret_cast<const VT*>(&v[V * p]);
         }
         for (int t = tid; t < 2 * c; t += bd) {
             const int sp = t / c, q = t % c;
@@ -677,9 +677,9 @@ bool sweep_ib_supported(int prec, int cplx, int ns, int nup, int ndn, int delay,
 int sweep_ib_fp64_delay(int cplx, int ns, int nup, int ndn, int nb) {
     // Fewer flushes against LDS (walkers per CU) and the terms a measurement
     // reads.  us of sweep kernel per N sweeps at delays 8 and 12: 216 rows
-    // 9003, 7041 (74090 with immediate updates); 150 rows 1103, 1154; 96 rows
-    // 689, 664, its local energies 97, 117 (2563 and 80 immediate).  Complex:
-    // 4 is slower everywhere (96 rows 1910 against 1376; 4371 immediate).
+    // 9003, 7041 (74090 with immediate updates), its local energies 182, 230;
+    // 150 rows 1103, 1154; 96 rows 689, 664 (2563 immediate).  Complex: 4 is
+    // slower everywhere (96 rows 1910 against 1376; 4371 immediate).
     const int d = !cplx && w_nsa(ns, nup, ndn) > 192 ? 12 : 8;
     return sweep_ib_supported(0, cplx, ns, nup, ndn, d, nb) ? d : 1;
 }

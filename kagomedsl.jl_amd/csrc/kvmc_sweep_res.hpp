@@ -142,7 +142,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
     constexpr int V = 16 / (int)sizeof(T), NVC = (DMAX + V - 1) / V;
     using VT = typename VecT<T, V>::type;
     if (c > 0) {
-        // pending terms: [spin][row][dp] and [spin][label][dp] in HBM
+        // pending terms: planes over rows and labels in HBM (pend_at)
         const int dp = pend_ld(delay);
         const T* gA = reinterpret_cast<const T*>(a.A) + (size_t)w * 2 * nsa * dp;
         const T* gB = reinterpret_cast<const T*>(a.Bm) + (size_t)w * 2 * a.nmax * dp;
@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                 VT v[NVC];
 #pragma unroll
                 for (int p = 0; p < NVC; ++p)
-                    if (V * p < c) v[p] = *reinterpret_cast<const VT*>(g + (size_t)lane * dp + V * p);
+                    if (V * p < c) v[p] = reinterpret_cast<const VT*>(g)[p * n + lane];
 #pragma unroll
                 for (int p = 0; p < NVC; ++p) {
                     const T* e = reinterpret_cast<const T*>(&v[p]);
@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
                         T* e = reinterpret_cast<T*>(&v);
 #pragma unroll
                         for (int u = 0; u < V; ++u) e[u] = V * p + u < c ? d[(V * p + u) * st + lane] : T(0);
-                        *reinterpret_cast<VT*>(g + (size_t)lane * dp + V * p) = v;
+                        reinterpret_cast<VT*>(g)[p * (part < 2 ? nsa : a.nmax) + lane] = v;
                     }
                 }
             }
