@@ -288,6 +288,7 @@ k_sweep_ib(SweepArgs a) {
     const long long stop = a.stop[w];
     if (sweeps >= stop || *a.failed != 0x7fffffff) return;
     int c = a.npend[w];
+    const int c_in = c;
     int acc_since = a.acc_since[w];
     // FP64: a walker whose last refresh found a nearly singular tildeU (its W
     // is large, and an update cancels most of its digits) updates W at once:
@@ -591,17 +592,24 @@ k_sweep_ib(SweepArgs a) {
     }
     __syncthreads();
     const auto k = late_args();
-    int* const slot_o = k->slot + (size_t)w * 2 * ns;
-    for (int t = tid; t < ns; t += bd) {
-        k->kup[(size_t)w * ns + t] = s_kup[t];
-        k->kdn[(size_t)w * ns + t] = s_kdn[t];
-        slot_o[t] = s_slu[t];
-        slot_o[ns + t] = s_sld[t];
+    if (n_acc) {
+        int* const slot_o = k->slot + (size_t)w * 2 * ns;
+        for (int t = tid; t < ns; t += bd) {
+            k->kup[(size_t)w * ns + t] = s_kup[t];
+            k->kdn[(size_t)w * ns + t] = s_kdn[t];
+            slot_o[t] = s_slu[t];
+            slot_o[ns + t] = s_sld[t];
+        }
     }
     // the terms are kept also for a walker due a refresh: the refresh may
     // measure the drift of the carried W first, and a walker whose refresh
-    // fails keeps a W consistent with its configuration
-    if (c > 0) {
+    // fails keeps a W consistent with its configuration.  Without an accepted
+    // move they are in memory as they were, and without a flush so are the
+    // rows of the terms that the launch began with (a call of one sweep, FP64,
+    // 8192 walkers at 216 rows: 831 us with all of them gathered and written,
+    // 336 now; at 96 rows 255 and 130).
+    if (c > 0 && n_acc) {
+        const int q0 = n_flush ? 0 : c_in / V * V;   // planes of rows before it are left
         T* gA = reinterpret_cast<T*>(k->A) + (size_t)w * 2 * nsa * dp;
         T* gB = reinterpret_cast<T*>(k->Bm) + (size_t)w * 2 * nmax * dp;
         int* pt = k->pterm + (size_t)w * 2 * kMaxDelay * 2;
@@ -631,11 +639,11 @@ k_sweep_ib(SweepArgs a) {
             __align__(16) T v[V * NVC];
 #pragma unroll
             for (int q = 0; q < V * NVC; ++q)
-                v[q] = q < c ? col[s_K[sp * kMaxDelay + q]] - (l == s_L[sp * kMaxDelay + q] ? T(1) : T(0)) : T(0);
+                v[q] = q >= q0 && q < c ? col[s_K[sp * kMaxDelay + q]] - (l == s_L[sp * kMaxDelay + q] ? T(1) : T(0)) : T(0);
             VT* g = reinterpret_cast<VT*>(gB + (size_t)sp * nmax * dp) + l;
 #pragma unroll
             for (int p = 0; p < NVC; ++p)
-                if (V * p < c) g[p * nmax] = *reinterpret_cast<const VT*>(&v[V * p]);
+                if (V * p >= q0 && V * p < c) g[p * nmax] = *reinterpret_cast<const VT*>(&v[V * p]);
         }
         for (int t = tid; t < 2 * c; t += bd) {
             const int sp = t / c, q = t % c;
