@@ -77,12 +77,14 @@ def sweep_bytes(cnt, s, ns, nup, ndn, nw):
     holds the rows of the empty sites only (ns - N per spin; the occupied
     rows are unit rows), plus a site -> row map per spin.
 
-    flush:    read + write both W once          2 s ((ns - nup) nup + (ns - ndn) ndn)
+    pass:     read + write both W once          2 s ((ns - nup) nup + (ns - ndn) ndn)
+              (cnt["w_passes"]; the flushes of an FP64 handle with immediate
+              updates are its accepted moves, several of which share a pass)
     accepted: column l + row K of both W        s ((ns - nup) + (ns - ndn) + nup + ndn) = 2 s ns
     move:     two W gathers for the ratio       2 s
     launch:   kappa and row maps, load + store  2 * 2 * 2 * 4 ns"""
     rows = (ns - nup) * nup + (ns - ndn) * ndn
-    return (cnt["flushes"] * 2 * s * rows + cnt["accepted"] * 2 * s * ns
+    return (cnt["w_passes"] * 2 * s * rows + cnt["accepted"] * 2 * s * ns
             + cnt["moves"] * 2 * s + cnt["launches"] * nw * 32 * ns)
 
 
@@ -147,13 +149,14 @@ def timed_steps(nat, ham, ds, args, precision, label):
     sync()
     # graph replay needs profiling off: kernel times are then not split
     ds.profile(not args.graph)
-    tot = dict(sweeps=0, moves=0, accepted=0, refreshes=0, flushes=0, launches=0)
+    tot = dict(sweeps=0, moves=0, accepted=0, refreshes=0, flushes=0, launches=0, w_passes=0)
     nap = 0
     energies = []
     sync()
     t0 = time.perf_counter()
     for _ in range(args.steps):
         cnt, _ = ds.sweep(S)
+        cnt["w_passes"] = ds.w_passes()
         e, na = ds.measure()
         for key in tot:
             tot[key] += cnt[key]
@@ -172,6 +175,8 @@ def timed_steps(nat, ham, ds, args, precision, label):
     def rate(num, ms):
         return num / (ms * 1e-3) if ms > 0 else None
 
+    if (rate(b_sweep, prof["sweep_ms"]) or 0) > 1e9 * HBM_PEAK_GBS:
+        log(f"[{label}] the sweep's byte count exceeds what {HBM_PEAK_GBS:.0f} GB/s carry in its time")
     res = {
         "walker_sweeps_per_s": nw * S * args.steps / wall,
         "ms_per_step": 1e3 * wall / args.steps,
@@ -446,7 +451,7 @@ def run_mixed(args):
         with MixedBatch([(ham, nw, shp)], **kw) as one:
             t1, r1, prof = timed(one, profile=True)
         alone_total += t1
-        c1 = r1[0][0]
+        c1 = dict(r1[0][0], w_passes=r1[0][0]["flushes"])   # delay > 1: every flush is a pass
         s = 8   # complex float W elements
         b = sweep_bytes(c1, s, ham.ns, ham.N_up, ham.N_down, nw)
         sweep_gbs = b / (prof[0]["sweep_ms"] * 1e-3) / 1e9 if prof[0]["sweep_ms"] > 0 else None

@@ -96,7 +96,8 @@ typedef struct kvmc_desc {
                                FP32 and FP64 alike.  FP64 handles may keep
                                terms of their own for immediate updates: the
                                same W to rounding, and each accepted move
-                               counts as a flush */
+                               counts as a flush (kvmc_get_w_passes has the
+                               updates of W in memory) */
     int32_t threads;        /* threads per workgroup of the sweep kernel (0: auto) */
     uint64_t seed;          /* Philox key of the device RNG */
     int32_t orbitals;       /* KVMC_ORB_* */
@@ -107,7 +108,7 @@ typedef struct kvmc_counters {
     int64_t moves;       /* proposals that reached the ratio (passed both early returns) */
     int64_t accepted;    /* accepted moves */
     int64_t refreshes;   /* walker refreshes (both spins) */
-    int64_t flushes;     /* delayed-update flushes */
+    int64_t flushes;     /* delayed-update flushes (delay <= 1: accepted moves) */
     int64_t launches;    /* sweep-kernel launches */
 } kvmc_counters;
 
@@ -153,6 +154,12 @@ int kvmc_refresh(kvmc_handle* h);
  * per sweep.  counters (optional) receives this call's totals. */
 int kvmc_sweep(kvmc_handle* h, int64_t nsweeps, const double* tape_u, const int32_t* tape_bond,
                int8_t* outcomes, kvmc_counters* counters);
+
+/* Times that the last sweep call of the handle read and wrote both W of a
+ * walker, summed over walkers: the flushes of pending terms, also of those an
+ * FP64 handle keeps for immediate updates, whose `flushes` are its accepted
+ * moves.  For byte counts; no counterpart in the reference. */
+int kvmc_get_w_passes(kvmc_handle* h, int64_t* passes);
 
 /* No counterpart in the reference.  kvmc_sweep for callers that cannot
  * allocate device memory (serving loops, harnesses that forbid allocation):

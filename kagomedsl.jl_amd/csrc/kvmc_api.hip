@@ -312,6 +312,7 @@ struct kvmc_handle {
     HostBlock* host = nullptr;                // pinned, written by kernels
     double* host_e = nullptr;                 // pinned [2 nw]: energies (re, im), log-determinants
     double* host_o = nullptr;                 // pinned: log-derivatives
+    int64_t w_passes = 0;                     // CNT_FLUSHES of the last sweep call
     int* nap = nullptr;                       // [nw] antiparallel bonds of the last measurement
     double* logdet = nullptr;
     double* eloc = nullptr;
@@ -947,6 +948,7 @@ int sweep_tail(kvmc_handle* h, const SweepArgs& a, int threads, size_t lds, bool
                      hipStreamSynchronize(s) != hipSuccess))
         return fail(KVMC_ERR_HIP, "outcome copy failed");
     const unsigned long long* cnt = h->host->total;
+    h->w_passes = (int64_t)cnt[CNT_FLUSHES];
     if (counters) {
         counters->sweeps = (int64_t)cnt[CNT_SWEEPS];
         counters->moves = (int64_t)cnt[CNT_MOVES];
@@ -1340,6 +1342,13 @@ int kvmc_get_w(kvmc_handle* h, int64_t walker, int32_t spin, double* out) {
                 out[cw * (l * ns + r) + p] = (sl[r] >= 0 && (size_t)sl[r] < ld)
                                                  ? rows[cw * (l * ld + sl[r]) + p]
                                                  : (p == 0 && kap[r] == (int)l + 1 ? 1.0 : 0.0);
+    return KVMC_OK;
+}
+
+int kvmc_get_w_passes(kvmc_handle* h, int64_t* passes) {
+    g_err.clear();
+    if (!h || !passes) return fail(KVMC_ERR_INVALID, "null argument");
+    *passes = h->w_passes;
     return KVMC_OK;
 }
 

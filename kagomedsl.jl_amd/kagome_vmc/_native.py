@@ -27,7 +27,7 @@ EXPORTS = [
     "kvmc_get_sweep_count", "kvmc_w_drift", "kvmc_failed_walker", "kvmc_last_error",
     "kvmc_version", "kvmc_profile_enable", "kvmc_get_profile", "kvmc_stagger_refresh",
     "kvmc_enable_graph", "kvmc_track_drift", "kvmc_get_drift_stats", "kvmc_sweep_noalloc",
-    "kvmc_group_create", "kvmc_group_sweep", "kvmc_group_destroy",
+    "kvmc_group_create", "kvmc_group_sweep", "kvmc_group_destroy", "kvmc_get_w_passes",
 ]
 
 
@@ -100,6 +100,7 @@ def load(path: str = LIB_PATH):
         "kvmc_measure_grad": ([vp, vp, vp], C.c_int),
         "kvmc_get_logdet": ([vp, vp], C.c_int),
         "kvmc_get_w": ([vp, C.c_int64, C.c_int32, vp], C.c_int),
+        "kvmc_get_w_passes": ([vp, P(C.c_int64)], C.c_int),
         "kvmc_set_sweep_count": ([vp, C.c_int64], C.c_int),
         "kvmc_get_sweep_count": ([vp, vp], C.c_int),
         "kvmc_w_drift": ([vp, P(C.c_double)], C.c_int),
@@ -224,6 +225,13 @@ class DeviceSampler:
         fn = load().kvmc_sweep_noalloc if noalloc else load().kvmc_sweep
         _check(fn(self._h, int(nsweeps), _ptr(tu), _ptr(tb), _ptr(out), C.byref(cnt)))
         return cnt.as_dict(), out
+
+    def w_passes(self):
+        """Reads and writes of a walker's W in the last sweep call, summed
+        over walkers (kvmc_get_w_passes)."""
+        n = C.c_int64(0)
+        _check(load().kvmc_get_w_passes(self._h, C.byref(n)))
+        return n.value
 
     def measure(self):
         """Per-walker local energies (FP64) and the antiparallel-bond count."""
