@@ -25,8 +25,7 @@
 //   (v_mfma_f64_16x16x4f64); then k_refresh_solve2, the solve with its tiles
 //   split over two wavefronts.
 //
-// N > 512 (or more sites than the solves' LDS takes): one kernel,
-// k_refresh_blocked<FULL = true>, which factors the tall matrix [tildeU ;
+// N > 512: one kernel, k_refresh_blocked<FULL = true>, which factors the tall matrix [tildeU ;
 // U_empty] (rows >= N end as L2 = U_empty U1^-1), solves X L1 = L2 panel by
 // panel and writes W_empty = X P through LDS.
 #include "kvmc_internal.hpp"
@@ -190,33 +189,6 @@ __device__ __forceinline__ double rcp_f64(double x) {
     double r = __builtin_amdgcn_rcp(x);
     r = fma(r, fma(-x, r, 1.0), r);
     return fma(r, fma(-x, r, 1.0), r);
-}
-
-// 16 x 16 diagonal blocks at (off, off) of the same inverses, for the
-// two-kernel path, one block per wavefront: lanes 0..15 of wavefront `wv`
-// each hold one column.  Rows >= jb of the block are unit rows.
-__device__ __attribute__((noinline)) void unit_lower_inverse16(const double* L, double* Linv, int off, int jb, int wv) {
-    if ((int)threadIdx.x / 64 != wv) return;
-    const int j = (int)threadIdx.x & 15;
-    double x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        double v = (i == j) ? 1.0 : 0.0;
-        if (i > j && off + i < jb) {
-            double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-            for (int k = 0; k < i; k += 2) {
-                s0 += L[(off + i) * LB + off + k] * x[k];
-                if (k + 1 < i) s1 += L[(off + i) * LB + off + k + 1] * x[k + 1];
-            }
-            v = -(s0 + s1);
-        }
-        x[i] = v;
-    }
-    if ((threadIdx.x & 63) < 16) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) Linv[(off + i) * LB + off + j] = x[i];
-    }
 }
 
 // Maximum of a 32-bit value over the wavefront, uniform result.
@@ -859,8 +831,11 @@ __global__ void __launch_bounds__(64 * LUW) __attribute__((amdgpu_waves_per_eu(N
     }
 }
 
-template <typename T, int RPT, bool FULL>
+// Above 256 labels: LU of tildeU alone for k_refresh_solve2 (FULL false, up to
+// 512 labels), or the whole refresh (FULL, up to 768).
+template <typename T, bool FULL>
 __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_refresh_blocked(RefreshArgs a) {
+    constexpr int RPT = FULL ? 3 : 2;   // panel rows per thread
     extern __shared__ __align__(16) unsigned char lds[];
     const int job = (int)blockIdx.x;
     if (job >= a.njobs) return;
@@ -1111,13 +1086,13 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
         const int c0 = j0 + RB;
         if (c0 >= nc16) continue;
         // U12 = L11^-1 A12 on MFMA: one 16-column block per wavefront at a
-        // time.  The single kernel at one or two panel rows per thread (two
-        // waves per SIMD) loads the next block's A12 operands while the
-        // current one is formed (bofs: the rows' offsets in U in the first
-        // panel, -1 for padding rows, in M afterwards); elsewhere that
-        // spills, and the operands are loaded per block.
+        // time.  With two panel rows per thread the next block's A12
+        // operands are loaded while the current one is formed (bofs: the
+        // rows' offsets in U in the first panel, -1 for padding rows, in M
+        // afterwards); with three that spills, and the operands are loaded
+        // per block.
         const int ntc = (nc16 - c0) / 16;
-        if constexpr (RPT <= 2) {
+        if constexpr (!FULL) {
             int bofs[RB / 4];
 #pragma unroll
             for (int s = 0; s < RB / 4; ++s) {
@@ -1181,12 +1156,12 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(2))) k_
         // (read back from M through L2; staged in LDS they took 102 KB at
         // N = 432, one workgroup per CU) feeds TG MFMA chains, and the next
         // column tile's operands are loaded while the current one is
-        // updated.  TG = 2 needs about 200 VGPRs: it fits the single kernel at
-        // two panel rows per thread (two waves per SIMD, under the panel's
-        // register peak) and spills elsewhere.  The C operands come from U in
+        // updated.  TG = 2 needs about 200 VGPRs: it fits with two panel
+        // rows per thread (two waves per SIMD, under the panel's register
+        // peak) and spills with three.  The C operands come from U in
         // the first panel and from M afterwards, a loop for each, so that
         // only one set of row offsets is live.
-        constexpr int TG = RPT == 2 ? 2 : 1;
+        constexpr int TG = FULL ? 1 : 2;
         const int r0 = c0;
         const int ntu = (nr16 - r0) / 16;
         int uofs[RB / 4];   // U12 operand rows: offsets in M
@@ -2077,11 +2052,11 @@ static hipError_t set_lds_limit(const void* fn, size_t lds) {
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
 }
 
-template <typename T, int RPT, bool FULL = true>
-static hipError_t launch_single(const RefreshArgs& a, size_t lds, hipStream_t s) {
-    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, RPT, FULL>), lds);
+template <typename T, bool FULL>
+static hipError_t launch_blocked(const RefreshArgs& a, size_t lds, hipStream_t s) {
+    hipError_t e = set_lds_limit(reinterpret_cast<const void*>(&k_refresh_blocked<T, FULL>), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL((k_refresh_blocked<T, RPT, FULL>), dim3(a.njobs), dim3(RT), lds, s, a);
+    hipLaunchKernelGGL((k_refresh_blocked<T, FULL>), dim3(a.njobs), dim3(RT), lds, s, a);
     return hipGetLastError();
 }
 
@@ -2112,14 +2087,6 @@ static hipError_t launch_solve(const RefreshArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Register tiles per wavefront of the solve kernel, or 0 for the
-// single-kernel path (N > 256, or LDS beyond 160 KiB).
-static int solve_tiles(int ns, int nmax) {
-    const int NT = solve_nt(nmax);
-    if (NT == 0 || solve_static_lds(NT) + solve_lds_bytes(ns, NT) > 160 * 1024) return 0;
-    return NT;
-}
-
 static size_t solve2_lds_bytes(int ns_out, int nb) { return (size_t)(nb * RB + 8 + ns_out) * sizeof(int); }
 
 template <typename T, int NB>
@@ -2134,16 +2101,11 @@ static hipError_t launch_solve2(const RefreshArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// 32-label blocks of k_refresh_solve2 for 256 < N <= 512, an even number, or 0.
-static int solve2_blocks(int ns, int nmax) {
-    const int nb = rup_i(refresh_npanel(nmax), 2);
-    return nmax > 256 && nb <= 16 && 48 * 1024 + solve2_lds_bytes(ns, nb) <= 160 * 1024 ? nb : 0;
-}
-
+// Every site holds one electron, so that there are at most 2 nmax sites: the
+// solves' LDS (73 KB at 256 labels, 55 KB at 512) always fits.
 template <typename T>
 static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t s) {
-    const int tiles = solve_tiles(a.ns, a.nmax);
-    if (tiles) {
+    if (a.nmax <= 256) {
         hipError_t e;
         switch (refresh_npanel(a.nmax)) {   // one instance per number of panels: tiles past the rows cost their products
             case 0: case 1: case 2: e = launch_lu<2, 2>(a, s); break;
@@ -2155,7 +2117,7 @@ static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t
             default: e = launch_lu<8, 2>(a, s); break;
         }
         if (e != hipSuccess) return e;
-        switch (tiles) {
+        switch (solve_nt(a.nmax)) {
             case 2: return launch_solve<T, 2>(a, s);
             case 4: return launch_solve<T, 4>(a, s);
             case 6: return launch_solve<T, 6>(a, s);
@@ -2168,22 +2130,17 @@ static hipError_t launch_refresh_t(const RefreshArgs& a, size_t lds, hipStream_t
     }
     // from 257 to 512 labels two kernels, measured 13.9 against 9.7 ms at 432;
     // beyond, half the tiles no longer fit a wavefront's registers
-    if (solve2_blocks(a.ns, a.nmax)) {
-        hipError_t e = launch_single<T, 2, false>(a, lds, s);
+    if (a.nmax <= 512) {
+        hipError_t e = launch_blocked<T, false>(a, lds, s);
         if (e != hipSuccess) return e;
-        switch (solve2_blocks(a.ns, a.nmax)) {
+        switch (rup_i(refresh_npanel(a.nmax), 2)) {   // 32-label blocks, an even number
             case 10: return launch_solve2<T, 10>(a, s);
             case 12: return launch_solve2<T, 12>(a, s);
             case 14: return launch_solve2<T, 14>(a, s);
             default: return launch_solve2<T, 16>(a, s);
         }
     }
-    switch (refresh_rows_per_thread(a.nmax)) {
-        case 1: return launch_single<T, 1>(a, lds, s);
-        case 2: return launch_single<T, 2>(a, lds, s);
-        case 3: return launch_single<T, 3>(a, lds, s);
-        default: return hipErrorInvalidValue;   // rejected by refresh_supported
-    }
+    return launch_blocked<T, true>(a, lds, s);   // at most 768 labels (refresh_supported)
 }
 
 // At most three panel rows per thread (N <= 768, i.e. 2N <= 768 for the real
