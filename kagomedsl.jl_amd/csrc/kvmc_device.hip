@@ -16,7 +16,8 @@ size_t sweep_lds_bytes(size_t esize, int ns, int nup, int ndn, int delay, int nb
 
 hipError_t launch_sweep(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
     // small clusters: W in LDS, one wavefront per walker
-    if (sweep_resident(w_elem_bytes(prec, 0), a.ns, a.nup, a.ndn) && sweep_w1_fits(a.ns, a.nup, a.ndn))
+    const size_t es = w_elem_bytes(prec, 0);
+    if (sweep_resident(es, a.ns, a.nup, a.ndn) && sweep_w1_fits(es, a.ns, a.nup, a.ndn, a.delay, a.nb))
         return prec == 0 ? launch_w1<double>(a, nw, s) : launch_w1<float>(a, nw, s);
     // W streamed from HBM with columns of at most 256 rows and pending terms:
     // pending rows kept implicit (no row reads at an accept)

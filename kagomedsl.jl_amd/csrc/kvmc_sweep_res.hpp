@@ -19,11 +19,6 @@
 
 namespace kvmc {
 
-__host__ __device__ inline bool sweep_w1_fits(int ns, int nup, int ndn) {
-    const int nmax = nup > ndn ? nup : ndn;
-    return w_nsa(ns, nup, ndn) <= 64 && nmax <= 64 && ns <= 128;
-}
-
 // w += a * b of one element, as vmac does per element of its vectors.
 __device__ __forceinline__ void emac(float& w, float a, float b) { w += a * b; }
 __device__ __forceinline__ void emac(double& w, double a, double b) { w += a * b; }
@@ -78,12 +73,19 @@ __device__ __forceinline__ void copy_vec(f32x4* d, const f32x4* g, int n) {
     }
 }
 
-__host__ __device__ inline size_t sweep_w1_lds(size_t es, int ns, int nup, int ndn, int delay, int nb) {
+inline size_t sweep_w1_lds(size_t es, int ns, int nup, int ndn, int delay, int nb) {
     const int nmax = nup > ndn ? nup : ndn;
     const size_t nsp = (size_t)(ns + 3) / 4 * 4;
     return w_stride(ns, nup, ndn) * es                                          // W (whole 16-byte vectors)
            + 2 * (size_t)delay * ((size_t)w_nsa(ns, nup, ndn) + (nmax + 3) / 4 * 4) * es   // pending terms
            + 4 * nsp * sizeof(int16_t) + bond_table_bytes(ns, nb);
+}
+
+// A row and a label per lane; with thousands of bonds the LDS can exceed that
+// of k_sweep, which takes the handle then.
+inline bool sweep_w1_fits(size_t es, int ns, int nup, int ndn, int delay, int nb) {
+    const int nmax = nup > ndn ? nup : ndn;
+    return w_nsa(ns, nup, ndn) <= 64 && nmax <= 64 && ns <= 128 && sweep_w1_lds(es, ns, nup, ndn, delay, nb) <= 160 * 1024;
 }
 
 template <typename T, int DMAX>
