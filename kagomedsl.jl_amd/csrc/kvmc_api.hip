@@ -309,9 +309,9 @@ struct kvmc_handle {
     int* all_walkers = nullptr;
     unsigned long long* counters = nullptr;   // [nw][CNT_SLOTS] of the current sweep call
     unsigned long long* total = nullptr;      // [CNT_SLOTS + 1] their sums and that of nap while a kernel forms them
-    int* ticket = nullptr;                    // blocks done (last_block)
+    int* ticket = nullptr;                    // [2] blocks done (last_block) of k_collect and of k_collect_eloc
     HostBlock* host = nullptr;                // pinned, written by kernels
-    double* host_e = nullptr;                 // pinned [2 nw]: energies (re, im), log-determinants
+    double* host_e = nullptr;                 // pinned [4 nw]: energies (re, im), log-determinants
     double* host_o = nullptr;                 // pinned: log-derivatives
     int64_t w_passes = 0;                     // CNT_FLUSHES of the last sweep call
     int* nap = nullptr;                       // [nw] antiparallel bonds of the last measurement
@@ -667,9 +667,9 @@ static int create_handle(const kvmc_desc* d, kvmc_handle** out, bool own_terms) 
     ALLOC(h->sweeps, nw); ALLOC(h->stop, nw); ALLOC(h->tbase, nw);
     ALLOC(h->rlist, nw); ALLOC(h->rcount, 1); ALLOC(h->failed, 1); ALLOC(h->all_walkers, nw);
     ALLOC(h->counters, nw * CNT_SLOTS); ALLOC(h->total, (size_t)CNT_SLOTS + 1); ALLOC(h->nap, nw);
-    ALLOC(h->ticket, 1);
+    ALLOC(h->ticket, 2);
     if (hipHostMalloc(reinterpret_cast<void**>(&h->host), sizeof(HostBlock), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&h->host_e), 2 * nw * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc(reinterpret_cast<void**>(&h->host_e), 4 * nw * sizeof(double), hipHostMallocDefault) != hipSuccess) {
         free_all(h); delete h; return fail(KVMC_ERR_NOMEM, "hipHostMalloc of the result buffers failed");
     }
     ALLOC(h->logdet, 2 * nw); ALLOC(h->eloc, nw); ALLOC(h->drift, 2 * nw); ALLOC(h->dstats, 3);
@@ -755,7 +755,7 @@ static int create_handle(const kvmc_desc* d, kvmc_handle** out, bool own_terms) 
         hipMemsetAsync(h->logdet, 0, 2 * nw * sizeof(double), h->stream) != hipSuccess ||
         hipMemsetAsync(h->dstats, 0, 3 * sizeof(double), h->stream) != hipSuccess ||
         hipMemsetAsync(h->total, 0, (CNT_SLOTS + 1) * sizeof(unsigned long long), h->stream) != hipSuccess ||
-        hipMemsetAsync(h->ticket, 0, sizeof(int), h->stream) != hipSuccess ||
+        hipMemsetAsync(h->ticket, 0, 2 * sizeof(int), h->stream) != hipSuccess ||
         hipStreamSynchronize(h->stream) != hipSuccess) {
         free_all(h);
         delete h;
@@ -1214,7 +1214,7 @@ static ElocArgs eloc_args(kvmc_handle* h) {
 // after the stream has finished.
 static int collect_eloc(kvmc_handle* h) {
     hipLaunchKernelGGL(k_collect_eloc, dim3(std::min(64, (h->nw + 255) / 256)), dim3(256), 0, h->stream, h->eloc,
-                       h->cplx ? h->eloc_im : nullptr, h->nap, h->nw, h->total + CNT_SLOTS, h->ticket, h->host_e, h->host);
+                       h->cplx ? h->eloc_im : nullptr, h->nap, h->nw, h->total + CNT_SLOTS, h->ticket + 1, h->host_e, h->host);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(h->stream));
     return KVMC_OK;
@@ -1310,8 +1310,8 @@ int kvmc_measure_grad(kvmc_handle* h, double* eloc, double* o) {
 int kvmc_get_logdet(kvmc_handle* h, double* logdet) {
     g_err.clear();
     if (!h || !logdet) return fail(KVMC_ERR_INVALID, "null argument");
-    const double* two = h->host_e;
-    HIP_TRY(hipMemcpyAsync(h->host_e, h->logdet, 2 * sizeof(double) * h->nw, hipMemcpyDeviceToHost, h->stream));
+    double* const two = h->host_e + (size_t)2 * h->nw;   // beside the energies, which another thread may be reading
+    HIP_TRY(hipMemcpyAsync(two, h->logdet, 2 * sizeof(double) * h->nw, hipMemcpyDeviceToHost, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
     // complex orbitals: the real form's determinant is |det tildeU|^2
     const double f = h->cplx ? 0.5 : 1.0;
