@@ -98,7 +98,12 @@ typedef struct kvmc_desc {
                                same W to rounding, and each accepted move
                                counts as a flush (kvmc_get_w_passes has the
                                updates of W in memory) */
-    int32_t threads;        /* threads per workgroup of the sweep kernel (0: auto) */
+    int32_t threads;        /* threads per workgroup of the sweep kernel (0: auto).
+                               Used where the kernel leaves a choice: complex
+                               float W and W of more than 256 rows per spin
+                               that are streamed; the kernels of small
+                               clusters (W in LDS) and of the other streamed
+                               W have one size (kvmc_get_sweep_threads) */
     uint64_t seed;          /* Philox key of the device RNG */
     int32_t orbitals;       /* KVMC_ORB_* */
 } kvmc_desc;
@@ -160,6 +165,9 @@ int kvmc_sweep(kvmc_handle* h, int64_t nsweeps, const double* tape_u, const int3
  * FP64 handle keeps for immediate updates, whose `flushes` are its accepted
  * moves.  For byte counts; no counterpart in the reference. */
 int kvmc_get_w_passes(kvmc_handle* h, int64_t* passes);
+
+/* Threads per workgroup that the handle's sweeps run with. */
+int kvmc_get_sweep_threads(kvmc_handle* h, int32_t* threads);
 
 /* No counterpart in the reference.  kvmc_sweep for callers that cannot
  * allocate device memory (serving loops, harnesses that forbid allocation):

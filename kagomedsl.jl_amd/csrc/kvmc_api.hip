@@ -551,6 +551,14 @@ int sweep_threads(const kvmc_handle* h) {
     return std::min(t, 512);
 }
 
+// Threads per workgroup of the kernel that the handle's sweeps run on.
+int sweep_block(const kvmc_handle* h) {
+    if (sweep_w1_supported(h->prec, h->cplx, h->ns, h->nup, h->ndn, h->delay, h->nb)) return 64;
+    if (sweep_ib_supported(h->prec, h->cplx, h->ns, h->nup, h->ndn, h->delay, h->nb))
+        return sweep_ib_block(h->ns, h->nup, h->ndn);
+    return sweep_threads(h);
+}
+
 // Real or complex instantiation of each kernel family.
 hipError_t do_sweep(const kvmc_handle* h, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
     return h->cplx ? launch_sweep_c(h->prec, a, nw, threads, lds, s) : launch_sweep(h->prec, a, nw, threads, lds, s);
@@ -1359,6 +1367,13 @@ int kvmc_get_w_passes(kvmc_handle* h, int64_t* passes) {
     g_err.clear();
     if (!h || !passes) return fail(KVMC_ERR_INVALID, "null argument");
     *passes = h->w_passes;
+    return KVMC_OK;
+}
+
+int kvmc_get_sweep_threads(kvmc_handle* h, int32_t* threads) {
+    g_err.clear();
+    if (!h || !threads) return fail(KVMC_ERR_INVALID, "null argument");
+    *threads = sweep_block(h);
     return KVMC_OK;
 }
 

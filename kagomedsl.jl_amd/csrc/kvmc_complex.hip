@@ -10,8 +10,7 @@ namespace kvmc {
 
 hipError_t launch_sweep_c(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
     // small clusters: W in LDS, one wavefront per walker
-    const size_t es = w_elem_bytes(prec, 1);
-    if (sweep_resident(es, a.ns, a.nup, a.ndn) && sweep_w1_fits(es, a.ns, a.nup, a.ndn, a.delay, a.nb))
+    if (sweep_w1_supported(prec, 1, a.ns, a.nup, a.ndn, a.delay, a.nb))
         return prec == 0 ? launch_w1<cf64>(a, nw, s) : launch_w1<cf32>(a, nw, s);
     if (sweep_ib_supported(prec, 1, a.ns, a.nup, a.ndn, a.delay, a.nb)) return launch_sweep_ib(prec, 1, a, nw, s);
     // 16-byte vectors: two complex floats or one complex double

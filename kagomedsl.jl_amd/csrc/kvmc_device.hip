@@ -14,10 +14,14 @@ size_t sweep_lds_bytes(size_t esize, int ns, int nup, int ndn, int delay, int nb
            (sweep_resident(esize, ns, nup, ndn) ? w_stride(ns, nup, ndn) * esize : 0);
 }
 
+bool sweep_w1_supported(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb) {
+    const size_t es = w_elem_bytes(prec, cplx);
+    return sweep_resident(es, ns, nup, ndn) && sweep_w1_fits(es, ns, nup, ndn, delay, nb);
+}
+
 hipError_t launch_sweep(int prec, const SweepArgs& a, int nw, int threads, size_t lds, hipStream_t s) {
     // small clusters: W in LDS, one wavefront per walker
-    const size_t es = w_elem_bytes(prec, 0);
-    if (sweep_resident(es, a.ns, a.nup, a.ndn) && sweep_w1_fits(es, a.ns, a.nup, a.ndn, a.delay, a.nb))
+    if (sweep_w1_supported(prec, 0, a.ns, a.nup, a.ndn, a.delay, a.nb))
         return prec == 0 ? launch_w1<double>(a, nw, s) : launch_w1<float>(a, nw, s);
     // W streamed from HBM with columns of at most 256 rows and pending terms:
     // pending rows kept implicit (no row reads at an accept)

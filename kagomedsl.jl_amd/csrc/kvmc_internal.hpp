@@ -230,10 +230,13 @@ hipError_t launch_sweep(int prec, const SweepArgs& a, int nwalkers, int threads,
                         hipStream_t s);
 hipError_t launch_sweep_c(int prec, const SweepArgs& a, int nwalkers, int threads, size_t lds,
                           hipStream_t s);
+// Small clusters, W in LDS: one wavefront per walker (kvmc_sweep_res.hpp).
+bool sweep_w1_supported(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb);
 // Sweep with implicit pending rows (kvmc_sweep_ib.hip): W streamed from HBM,
 // at most 256 rows per spin, 1 < delay <= kMaxDelay (8 for complex W), real
-// FP32 or any FP64.
+// FP32 or any FP64; sweep_ib_block threads per workgroup.
 bool sweep_ib_supported(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb);
+int sweep_ib_block(int ns, int nup, int ndn);
 // The delay FP64 handles with immediate updates (delay <= 1) run with: the
 // same W to rounding, streamed once per that many accepts; 1 where the kernel
 // does not apply.

@@ -75,11 +75,6 @@ struct IbMove {
     int e[2], l[2];             // row of the target site, label
 };
 
-__host__ __device__ inline int sweep_ib_threads(int ns, int nup, int ndn) {
-    const int nsa = w_nsa(ns, nup, ndn);
-    return nsa <= 64 ? 64 : nsa <= 128 ? 128 : nsa <= 192 ? 192 : 256;
-}
-
 template <typename T>
 __host__ __device__ inline size_t sweep_ib_lds(int ns, int nsa, int nwave, int delay, int nb) {
     const size_t nsp = (size_t)(ns + 3) / 4 * 4;
@@ -668,8 +663,13 @@ k_sweep_ib(SweepArgs a) {
     }
 }
 
+int sweep_ib_block(int ns, int nup, int ndn) {
+    const int nsa = w_nsa(ns, nup, ndn);
+    return nsa <= 64 ? 64 : nsa <= 128 ? 128 : nsa <= 192 ? 192 : 256;
+}
+
 static size_t ib_lds(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb) {
-    const int nsa = w_nsa(ns, nup, ndn), nwave = sweep_ib_threads(ns, nup, ndn) / 64;
+    const int nsa = w_nsa(ns, nup, ndn), nwave = sweep_ib_block(ns, nup, ndn) / 64;
     if (prec == 1) return sweep_ib_lds<float>(ns, nsa, nwave, delay, nb);
     return cplx ? sweep_ib_lds<cf64>(ns, nsa, nwave, delay, nb) : sweep_ib_lds<double>(ns, nsa, nwave, delay, nb);
 }
@@ -699,7 +699,7 @@ static hipError_t launch_ib_d(const SweepArgs& a, int nw, size_t lds, hipStream_
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((k_sweep_ib<T, D, M, UNR, EX>), dim3(nw), dim3(sweep_ib_threads(a.ns, a.nup, a.ndn)), lds, s, a);
+    hipLaunchKernelGGL((k_sweep_ib<T, D, M, UNR, EX>), dim3(nw), dim3(sweep_ib_block(a.ns, a.nup, a.ndn)), lds, s, a);
     return hipGetLastError();
 }
 

@@ -28,6 +28,7 @@ EXPORTS = [
     "kvmc_version", "kvmc_profile_enable", "kvmc_get_profile", "kvmc_stagger_refresh",
     "kvmc_enable_graph", "kvmc_track_drift", "kvmc_get_drift_stats", "kvmc_sweep_noalloc",
     "kvmc_group_create", "kvmc_group_sweep", "kvmc_group_destroy", "kvmc_get_w_passes",
+    "kvmc_get_sweep_threads",
 ]
 
 
@@ -101,6 +102,7 @@ def load(path: str = LIB_PATH):
         "kvmc_get_logdet": ([vp, vp], C.c_int),
         "kvmc_get_w": ([vp, C.c_int64, C.c_int32, vp], C.c_int),
         "kvmc_get_w_passes": ([vp, P(C.c_int64)], C.c_int),
+        "kvmc_get_sweep_threads": ([vp, P(C.c_int32)], C.c_int),
         "kvmc_set_sweep_count": ([vp, C.c_int64], C.c_int),
         "kvmc_get_sweep_count": ([vp, vp], C.c_int),
         "kvmc_w_drift": ([vp, P(C.c_double)], C.c_int),
@@ -231,6 +233,13 @@ class DeviceSampler:
         over walkers (kvmc_get_w_passes)."""
         n = C.c_int64(0)
         _check(load().kvmc_get_w_passes(self._h, C.byref(n)))
+        return n.value
+
+    def sweep_threads(self):
+        """Threads per workgroup that the sweeps run with; `threads` is used
+        only where the kernel leaves a choice."""
+        n = C.c_int32(0)
+        _check(load().kvmc_get_sweep_threads(self._h, C.byref(n)))
         return n.value
 
     def measure(self):
