@@ -311,7 +311,7 @@ struct kvmc_handle {
     unsigned long long* total = nullptr;      // [CNT_SLOTS + 1] their sums and that of nap while a kernel forms them
     int* ticket = nullptr;                    // [2] blocks done (last_block) of k_collect and of k_collect_eloc
     HostBlock* host = nullptr;                // pinned, written by kernels
-    double* host_e = nullptr;                 // pinned [4 nw]: energies (re, im), log-determinants
+    double* host_e = nullptr;                 // behind host, [4 nw]: energies (re, im), log-determinants
     double* host_o = nullptr;                 // pinned: log-derivatives
     int64_t w_passes = 0;                     // CNT_FLUSHES of the last sweep call
     int* nap = nullptr;                       // [nw] antiparallel bonds of the last measurement
@@ -357,7 +357,7 @@ void free_all(kvmc_handle* h) {
                     h->logdet, h->eloc, h->drift, h->dstats, h->ws, h->Qup, h->Qdn, h->O};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
-    for (void* p : {(void*)h->host, (void*)h->host_e, (void*)h->host_o})
+    for (void* p : {(void*)h->host, (void*)h->host_o})
         if (p) (void)hipHostFree(p);
     if (h->ev0) (void)hipEventDestroy(h->ev0);
     if (h->ev1) (void)hipEventDestroy(h->ev1);
@@ -676,10 +676,14 @@ static int create_handle(const kvmc_desc* d, kvmc_handle** out, bool own_terms) 
     ALLOC(h->rlist, nw); ALLOC(h->rcount, 1); ALLOC(h->failed, 1); ALLOC(h->all_walkers, nw);
     ALLOC(h->counters, nw * CNT_SLOTS); ALLOC(h->total, (size_t)CNT_SLOTS + 1); ALLOC(h->nap, nw);
     ALLOC(h->ticket, 2);
-    if (hipHostMalloc(reinterpret_cast<void**>(&h->host), sizeof(HostBlock), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&h->host_e), 4 * nw * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    // one allocation: each costs about 50 us
+    if (hipHostMalloc(reinterpret_cast<void**>(&h->host), 256 + 4 * nw * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        h->host = nullptr;
         free_all(h); delete h; return fail(KVMC_ERR_NOMEM, "hipHostMalloc of the result buffers failed");
     }
+    static_assert(sizeof(HostBlock) <= 256, "the energies lie 256 bytes behind the block");
+    h->host_e = reinterpret_cast<double*>(reinterpret_cast<unsigned char*>(h->host) + 256);
     ALLOC(h->logdet, 2 * nw); ALLOC(h->eloc, nw); ALLOC(h->drift, 2 * nw); ALLOC(h->dstats, 3);
     // refresh workspace: up to 16 GiB of FP64 work matrices per batch (about
     // 10000 walkers at 432 sites, so one launch pair covers even a refresh of
