@@ -11,8 +11,9 @@ Forms (each its own handle):
   fp32       W in FP32 with `delay` pending rank-1 terms per flush, FP64 local
              energy, FP64 LU refresh every k accepted moves (EVERY_K: a walker
              is refreshed as soon as it reaches k)            -> `value`
-  fp64       the plain FP64 sampler: W in FP64, immediate rank-1 updates,
-             FP64 refresh every N accepted moves (EVERY_K, k = N)
+  fp64       the plain FP64 sampler: W in FP64, immediate rank-1 updates
+             (the library keeps them as pending terms: the same W to
+             rounding), FP64 refresh every N accepted moves (EVERY_K, k = N)
   fp64_ref   FP64 with the reference's refresh cadence (src/MonteCarlo.jl:
              593-604: every min(N_up, N_dn) sweeps that pass the early returns)
   fp32 k=... the FP32 form at the other refresh intervals
@@ -46,12 +47,12 @@ FP64_PEAK_TFLOPS = 78.6
 
 # HBM bytes (FETCH_SIZE + WRITE_SIZE, calibrated against a plain copy) per
 # walker refreshed by the kernel pair k_lu + k_refresh_solve, from
-# rocprofv3 --pmc passes over a refresh of 8192 walkers at L=12 (summary in
+# rocprofv3 --pmc passes over the default FP32 form at L=12 (summary in
 # profiles/).
-REFRESH_TRAFFIC_BYTES_PER_WALKER = {12: 5_548_823}
+REFRESH_TRAFFIC_BYTES_PER_WALKER = {12: 5_755_308}
 # the same for the FP32 sweep kernel (k_sweep_ib), per walker-sweep (delay 12,
 # L=12, refresh every 216 accepts)
-SWEEP_TRAFFIC_BYTES_PER_WALKER_SWEEP = {12: 10_394}
+SWEEP_TRAFFIC_BYTES_PER_WALKER_SWEEP = {12: 9_808}
 
 # closed-shell boundary conditions per cluster size
 BC = {4: ((True, True), (False, True)), 6: ((True, True), (False, False)),

@@ -1774,8 +1774,10 @@ k_refresh_solve(RefreshArgs a, int groups) {
 // SIMD).  The wavefront that holds block J forms y_J and hands it to its
 // partner through LDS, a step ahead: the block that comes next is updated
 // first and its y formed before the other updates.  The factors' rows are read
-// as operands straight from memory, 128 bytes a row, two blocks ahead; the
-// wavefronts of a workgroup read the same ones through L1.
+// as operands straight from memory, 128 bytes a row; the wavefronts of a
+// workgroup read the same ones through L1.  The first two blocks' operands of a
+// step are requested before its barrier, which waits for them all (it is
+// preceded by a wait for every load): each step exposes one memory latency.
 //
 // With an odd number of blocks the last tile pair reads what follows the rows (in
 // bounds: the inverses lie behind them); it is never a block of y.

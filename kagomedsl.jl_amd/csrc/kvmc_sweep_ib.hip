@@ -38,12 +38,12 @@
 //     needs of the column's term rows, so they are published with the move and
 //     an accept costs one load of the two columns and two barriers.
 //
-// Bound by HBM: the flushes' reads and writes of W, plus about 40 % more for
+// Bound by HBM: the flushes' reads and writes of W, plus about 30 % more for
 // the gathers, an accept's columns and the launch's ends.  Measured per N
-// sweeps of 8192 walkers at 216 rows: FP32, delay 12, 5.12 -> 4.28 ms (18.4 GB
-// counted before, 4.3 TB/s; a plain copy reaches 4.8); FP64 with immediate
-// updates asked for, 74.1 -> 7.0 ms (delay 12 inside).  4096 walkers at 96
-// rows, FP64: 2.56 -> 0.68 ms; 2048 at 96 rows, complex FP64: 4.37 -> 1.38 ms.
+// sweeps of 8192 walkers at 216 rows: FP32, delay 12, 5.12 -> 4.25 ms (17.4 GB
+// counted, 4.1 TB/s; a plain copy reaches 4.8); FP64 with immediate updates
+// asked for, 74.1 -> 7.0 ms (delay 12 inside).  4096 walkers at 96 rows, FP64:
+// 2.56 -> 0.68 ms; 2048 at 96 rows, complex FP64: 4.37 -> 1.38 ms.
 //
 // Between launches the pending terms are kept in the layout of k_sweep
 // (pend_at) with A = At and B = g, so the local energy, the flush kernel,
@@ -676,6 +676,10 @@ static size_t ib_lds(int prec, int cplx, int ns, int nup, int ndn, int delay, in
 
 bool sweep_ib_supported(int prec, int cplx, int ns, int nup, int ndn, int delay, int nb) {
     const int ld = w_ld(ns, nup) > w_ld(ns, ndn) ? w_ld(ns, nup) : w_ld(ns, ndn);
+    // complex: a lane holds the terms of 2 or 4 rows, 4 registers each, and
+    // more than 8 of them would spill.  Such delays run on k_sweep: us of sweep
+    // kernel per N sweeps there at 12 terms and here at 8, 1024 walkers at 96
+    // rows 740 and 541, 512 at 150 rows 1384 and 1067.
     const int dmax = prec == 0 && cplx ? 8 : kMaxDelay;
     if (prec == 1 && cplx) return false;
     return delay > 1 && delay <= dmax && ld <= 256 && !sweep_resident(w_elem_bytes(prec, cplx), ns, nup, ndn) &&
@@ -687,7 +691,9 @@ int sweep_ib_fp64_delay(int cplx, int ns, int nup, int ndn, int nb) {
     // reads.  us of sweep kernel per N sweeps at delays 8 and 12: 216 rows
     // 9003, 7041 (74090 with immediate updates), its local energies 182, 230;
     // 150 rows 1103, 1154; 96 rows 689, 664 (2563 immediate).  Complex: 4 is
-    // slower everywhere (96 rows 1910 against 1376; 4371 immediate).
+    // slower everywhere (96 rows 1910 against 1376, 4371 immediate; 216 rows,
+    // 512 walkers, 3306 against 2420, 11519 immediate; 150 rows 1065, 3216
+    // immediate), also where 8 terms spill 10 registers (above 128 rows).
     const int d = !cplx && w_nsa(ns, nup, ndn) > 192 ? 12 : 8;
     return sweep_ib_supported(0, cplx, ns, nup, ndn, d, nb) ? d : 1;
 }

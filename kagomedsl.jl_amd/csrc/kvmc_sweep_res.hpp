@@ -9,7 +9,8 @@
 //   - 64 draws are held in registers, one per lane, until they are passed;
 //   - Z_mu changes by one bond per lane, for the accepted move only (k_sweep
 //     walks the neighbours of every proposal);
-//   - nothing spills (k_sweep's instance for 12 terms spilled 89 registers).
+//   - no vector register spills (k_sweep's instance for 12 terms spilled 89);
+//     150 to 212 scalar ones do, into lanes of vector registers.
 // us of sweep kernels per N sweeps, k_sweep and here: 777 walkers of 108 sites,
 // FP64, 263 and 192; 4096 walkers of 48 sites, FP32, delay 12, 320 and 272 (96
 // with the counters kept per walker).
