@@ -24,7 +24,7 @@ def test_fp64_handle_without_room_for_its_own_terms():
     terms = nw * 2 * (12 - 4) * (216 + 216) * 8          # of 12 slots a row instead of 4
     assert terms > 400 << 20
     # the bulk, then steps of half of the terms until a handle that asks
-    # for 12 terms no longer fits (what the driver counts as free is not exact)
+    # for 12 terms no longer fits (the free memory that HIP reports is not exact)
     hold, full = [], False
     try:
         hold.append(torch.empty(free() - need - (1 << 30), dtype=torch.uint8, device="cuda"))
